@@ -1,0 +1,56 @@
+// The resident Krylov engine: a whole solve in one launch, every right-hand side (or segmented
+// piece) held by a team of workgroups with its matrix rows and vectors in registers. See
+// pp_resident.hip.
+#pragma once
+
+#include "pp_krylov.hpp"
+
+namespace pp {
+
+constexpr int RES_WG = 512;        // threads of a multi-workgroup team's workgroups
+constexpr int RES_LOCAL_WG = 1024; // threads at most of a one-workgroup team
+constexpr int RES_TOLS = 8;        // tolerances passed by value
+
+// Pieces of a segmented solve: piece k has len[k] rows at vector offset base[k], its matrix rows
+// start at mrow[k]; workgroup w works on piece wgPiece[w], whose workgroups are
+// wgOff[k] .. wgOff[k + 1] - 1. All null for a plain solve.
+struct ResPieces {
+    const int32_t *base, *len, *mrow, *wgPiece, *wgOff;
+};
+
+template <typename T>
+struct ResArgs {
+    Csr<T> A;
+    const T *b;
+    T *x, *xbest;                // xbest: null without return-best
+    const T *dinv;               // Jacobi preconditioner (null: none)
+    int dinvStride;
+    unsigned long long *zbuf;    // exchanged vectors: [2][vecLen] values in tagged words
+    unsigned long long *slots;   // partial sums: [2][3][wgs] values in tagged words
+    size_t vecLen, zorigin;      // values per parity; vector offset of the first of them
+    SolveRec *recs;              // final records
+    unsigned *status;            // per right-hand side: `done` from the team that finished it
+    unsigned *failed;            // `done` from a workgroup that gave up
+    unsigned tag, done;          // the exchanges' first tag less one; the launch's word
+    int n, rpm, G, team0;        // plain solve: rows, right-hand sides per matrix, workgroups per team, first team
+    int wgs;                     // workgroups of the launch
+    int maxit, returnBest, project, resetEvery;
+    int zeroStops;               // a zero right-hand side ends at once (x = 0)
+    double scale;                // 1 / sqrt(n) or 1 (a plain solve)
+    double tols[RES_TOLS];       // per right-hand side when tolsDev is null (one: tols[0])
+    int ntols;
+    const double *tolsDev;
+    ResPieces P;
+};
+
+// Largest one-workgroup system, in rows, for stencil rows of `ew` entries.
+inline int resident_local_rows(int ew) { return (ew == 5 ? 4 : 3) * RES_LOCAL_WG; }
+
+// Launch on `wgs` workgroups: local = every team is one workgroup of `threads` threads with up
+// to R rows per thread; otherwise teams of RES_WG-thread workgroups with R rows per thread.
+template <typename T>
+int launch_resident_cg(const ResArgs<T> &a, int ew, int R, int threads, bool local, hipStream_t s);
+template <typename T>
+int launch_resident_bicg(const ResArgs<T> &a, int ew, int R, int threads, bool local, hipStream_t s);
+
+} // namespace pp

@@ -18,7 +18,7 @@
 // Recurrences, stopping rules and reported iteration counts restate the reference's fused
 // solvers (csrc/phipict/solvers/krylov/krylov.cu: CG :291-568, BiCGStab :598-824, AMG-PCG
 // :1389-1546 with the V-cycle :1247-1385); the rules themselves are in pp_krylov.hpp.
-#include "pp_krylov.hpp"
+#include "pp_resident.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -1053,6 +1053,9 @@ struct Space {
     void *tailDev = nullptr; size_t tailCap = 0;
     void *tailHost = nullptr;
     char *snap = nullptr;  size_t snapCap = 0;  // pinned snapshots: two slots of B records
+    void *link = nullptr;  size_t linkCap = 0;  // tagged words of the resident engine, never anything else
+    uint32_t linkTag = 0;                       // the largest tag they may hold
+    unsigned solves = 0;                        // resident solves so far: their status word
     bool fixed = false;    // carved from the static scratch array: never grows, never freed
     hipEvent_t ev[2] = {nullptr, nullptr}; // snapshot events created once (fixed spaces)
 };
@@ -1541,6 +1544,146 @@ static int bicg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const
         return PP_OK;
     }
     report(slot_recs(sp, last, B), B, 0, res);
+    return PP_OK;
+}
+
+// ---------------- the resident engine ----------------
+// Launches with teams of several workgroups run one at a time: every member must be resident.
+static std::mutex g_resident_lock;
+
+// How a resident solve of `teams` systems of n rows runs: one workgroup each, or teams of G
+// workgroups with R rows per thread, `perLaunch` teams at a time. ew 0: not on this engine.
+//
+// Measured, us per CG iteration in FP64 (the multi-launch engine: 42 at 160 k rows, 36 at 105 k; the
+// one-workgroup engine: 24 at 4 k rows and growing with the rows):
+//   one workgroup:     1 k rows 1.7, 3 k 2.1, 4 k (five entries) 2.9, 3 k (seven) 2.5
+//   teams, R = 1:      4 k 3.9, 8 k 4.2, 31 k 4.8 (five); 31 k 5.0, 105 k 7.1 (seven)
+//   teams, R = 2:      8 k 4.6, 31 k 4.9; 31 k 5.8, 105 k 7.4, 160 k 8.7, 246 k 9.3
+//   teams, R = 4:      8 k 5.5, 31 k 6.8; 31 k 9.8, 105 k 11.9, 246 k 15
+// so one workgroup as long as its registers hold the rows, then the fewest rows per thread
+// that let all teams run at once; if none does, as many teams at a time as fit with R = 4.
+struct ResPlan {
+    int ew = 0, R = 0, threads = 0, G = 1, perLaunch = 0;
+    bool local = false;
+};
+
+// Entries per row the kernels are built for: the ELL width, or for plain CSR a guess from the
+// mean row length, which the kernel checks against every row.
+template <typename T>
+static int resident_width(const Csr<T> &A, long nnz) {
+    if (A.ell_w > 0) return A.ell_w == 5 || A.ell_w == 7 ? A.ell_w : 0;
+    return nnz <= 5l * A.n ? 5 : (nnz <= 7l * A.n ? 7 : 0);
+}
+
+static ResPlan resident_plan(int n, int teams, int ew) {
+    ResPlan p;
+    if (!ew) return p;
+    if (n <= resident_local_rows(ew)) {
+        p.local = true;
+        p.R = (n + RES_LOCAL_WG - 1) / RES_LOCAL_WG;
+        p.threads = std::min(RES_LOCAL_WG, (n + 63) / 64 * 64); // rows dealt out as by the one-workgroup engine
+        p.perLaunch = teams;
+        p.ew = ew;
+        return p;
+    }
+    const int cus = std::min(cu_count(), RES_WG);
+    for (int R : {1, 2, 4}) {
+        const int G = (n + RES_WG * R - 1) / (RES_WG * R);
+        const int fit = cus / G;
+        if (fit >= teams || (R == 4 && fit > 0)) {
+            p.R = R;
+            p.G = G;
+            p.threads = RES_WG;
+            p.perLaunch = std::min(fit, teams);
+            p.ew = ew;
+            return p;
+        }
+    }
+    return p;
+}
+
+// `words` tagged words whose tags are at most *tag, with room for `tags` more.
+static int resident_link(Space &sp, size_t words, uint32_t tags, hipStream_t s, uint32_t *tag) {
+    const size_t bytes = words * sizeof(uint64_t);
+    if (sp.fixed) PP_CHECK_ARG(bytes <= sp.linkCap, "solve exceeds the static exchange buffer");
+    const bool grown = sp.linkCap < bytes;
+    if (int e = grown ? grow(&sp.link, &sp.linkCap, bytes) : PP_OK) return e;
+    if (grown || sp.linkTag > UINT32_MAX - tags) {
+        hipLaunchKernelGGL((k_fill_zero<double>), dim3(1024), dim3(256), 0, s, reinterpret_cast<double *>(sp.link),
+                           sp.linkCap / sizeof(double));
+        PP_LAUNCH_CHECK();
+        sp.linkTag = 0;
+    }
+    *tag = sp.linkTag;
+    return PP_OK;
+}
+
+constexpr int RES_MAXIT = 1 << 26; // above it the tags of one solve could wrap
+
+// *ran: the engine finished the solve (false: run another engine; x holds a start guess).
+template <typename T>
+static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x, int B, int maxit, const double *tols,
+                          int ntols, double scale, int resetEvery, int returnBest, int project, int bicg, int jacobi,
+                          int zeroStops, Space &sp, hipStream_t s, const SolveRec **recs, bool *ran) {
+    const int n = A.n;
+    *ran = false;
+    const int numMat = (B + A.rpm - 1) / A.rpm;
+    const size_t len = (size_t)n * B;
+    if (int e = prepare(sp, sizeof(T) * (len + (size_t)numMat * n), 8, B, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
+    T *xbest = reinterpret_cast<T *>(sp.vec);
+    T *dinv = jacobi ? xbest + len : nullptr;
+    if (jacobi) launch_jacobi<T>(A, numMat, dinv, s);
+    ResArgs<T> a{};
+    a.A = A;
+    a.b = b; a.x = x; a.xbest = returnBest ? xbest : nullptr;
+    a.dinv = dinv; a.dinvStride = A.valStride ? n : 0;
+    a.vecLen = (size_t)n * plan.perLaunch;
+    a.n = n; a.rpm = A.rpm; a.G = plan.G;
+    a.maxit = maxit; a.returnBest = returnBest; a.project = project; a.resetEvery = resetEvery; a.zeroStops = zeroStops;
+    a.scale = scale;
+    a.ntols = ntols > RES_TOLS ? 1 : ntols;
+    for (int k = 0; k < a.ntols; ++k) a.tols[k] = tols[k];
+    a.tolsDev = ntols > RES_TOLS ? (const double *)sp.tols : nullptr;
+    const int maxWgs = plan.perLaunch * plan.G;
+    const size_t zWords = plan.local ? 0 : 2 * a.vecLen * (sizeof(T) / 4), slotWords = plan.local ? 0 : (size_t)2 * 3 * maxWgs * 2;
+    // exchanges of one launch at most: two sums per iteration, two more words per residual replacement
+    const uint32_t tags = (uint32_t)(4 * ((int64_t)maxit + 4));
+    const int launches = (B + plan.perLaunch - 1) / plan.perLaunch;
+    if (!plan.local && (uint64_t)tags * launches > (1u << 31)) return PP_OK;
+    std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
+    if (!plan.local) alone.lock();
+    if (!plan.local) {
+        uint32_t tag = 0;
+        if (int e = resident_link(sp, zWords + slotWords, tags * (uint32_t)launches, s, &tag)) return e;
+        a.zbuf = reinterpret_cast<unsigned long long *>(sp.link);
+        a.slots = a.zbuf + zWords;
+        a.tag = tag;
+    }
+    // the records, then (in the second copy's place) a word per team and one for failures, come
+    // back in one copy; the words of this solve are told from older contents by their value
+    a.recs = recs_a(sp);
+    a.status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
+    a.failed = a.status + B;
+    a.done = 0xC0DE0000u + (++sp.solves & 0xffffu);
+    for (int t0 = 0; t0 < B; t0 += plan.perLaunch) {
+        const int teams = std::min(plan.perLaunch, B - t0);
+        a.team0 = t0;
+        a.zorigin = (size_t)t0 * n;
+        a.wgs = teams * plan.G;
+        int e = PP_OK;
+        PP_TIMED(bicg ? PP_K_BICG_SMALL : PP_K_CG_SMALL, n, s,
+                 e = launch_resident_cg<T>(a, plan.ew, plan.R, plan.threads, plan.local, s));
+        if (e) return e;
+        a.tag += tags;
+        sp.linkTag += plan.local ? 0 : tags;
+    }
+    char *host = sp.snap;
+    PP_HIP(hipMemcpyAsync(host, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 1), hipMemcpyDeviceToHost, s));
+    PP_HIP(hipStreamSynchronize(s));
+    *recs = reinterpret_cast<const SolveRec *>(host);
+    const unsigned *st = reinterpret_cast<const unsigned *>(host + sizeof(SolveRec) * B);
+    *ran = st[B] != a.done;
+    for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
     return PP_OK;
 }
 
@@ -2412,7 +2555,30 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
         const T *b = reinterpret_cast<const T *>(rhs);
         T *xx = reinterpret_cast<T *>(x);
         Space &sp = use_bicg ? bicgSpace : cgSpace;
-        if (A->n <= SMALL_N)
+        const bool small = A->n <= SMALL_N;
+        const ResPlan plan = use_bicg ? ResPlan{} : resident_plan(A->n, nrhs, resident_width<T>(C, A->nnz));
+        if (plan.ew && maxit <= RES_MAXIT && (small || plan.perLaunch >= nrhs)) {
+            const SolveRec *recs = nullptr;
+            bool ran = false;
+            if (int e = resident_solve<T>(C, plan, b, xx, nrhs, maxit, tols, ntols, scale,
+                                          use_bicg ? 0 : residual_reset_steps, return_best, matrix_rank_deficient, use_bicg,
+                                          jacobi, !small && nrhs == 1, sp, s, &recs, &ran))
+                return e;
+            if (ran) {
+                if (!small && all_zero_rhs(recs, nrhs)) {
+                    if (nrhs > 1) {
+                        hipLaunchKernelGGL((k_fill_zero<T>), dim3(std::min(4096, (A->n * nrhs + 255) / 256)), dim3(256), 0,
+                                           s, xx, (size_t)A->n * nrhs);
+                        PP_LAUNCH_CHECK();
+                    }
+                    report_zero(nrhs, results);
+                } else {
+                    report(recs, nrhs, return_best, results);
+                }
+                return PP_OK;
+            }
+        }
+        if (small)
             return small_solve<T>(C, b, xx, nrhs, maxit, tols, ntols, scale, use_bicg ? 0 : residual_reset_steps,
                                   return_best, matrix_rank_deficient, use_bicg, jacobi, sp, s, results);
         if (use_bicg) return bicg_large<T>(C, b, xx, nrhs, maxit, tols, ntols, scale, jacobi, sp, s, results);
@@ -2429,7 +2595,8 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
 // array and the snapshot events are created at that set-up too.
 constexpr size_t SCR_VEC = size_t(56) << 20, SCR_PARTS = size_t(6) << 20, SCR_RECS = size_t(1) << 20,
                  SCR_TOLS = size_t(64) << 10;
-constexpr size_t SCRATCH_BYTES = SCR_VEC + SCR_PARTS + SCR_RECS + SCR_TOLS;
+constexpr size_t SCR_LINK = size_t(20) << 20; // tagged words of the resident engine: 262144 doubles and their sums
+constexpr size_t SCRATCH_BYTES = SCR_VEC + SCR_PARTS + SCR_RECS + SCR_TOLS + SCR_LINK;
 constexpr int SCRATCH_RHS = 2048;     // right-hand sides per call at most
 constexpr int SCRATCH_DEVICES = 16;   // devices of one process with a scratch table entry
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
@@ -2450,6 +2617,7 @@ static int fixed_space(Space **out) {
         sp.parts = base + SCR_VEC;                        sp.partsCap = SCR_PARTS;
         sp.recs = base + SCR_VEC + SCR_PARTS;             sp.recsCap = SCR_RECS;
         sp.tols = base + SCR_VEC + SCR_PARTS + SCR_RECS;  sp.tolsCap = SCR_TOLS;
+        sp.link = base + SCR_VEC + SCR_PARTS + SCR_RECS + SCR_TOLS; sp.linkCap = SCR_LINK;
         sp.snap = reinterpret_cast<char *>(g_fixed_snap); sp.snapCap = sizeof(g_fixed_snap);
         sp.fixed = true;
     }
@@ -2593,7 +2761,7 @@ int pp_release_workspaces(void) {
         ts->tbuf = nullptr; ts->tbad = nullptr; ts->tcap = 0;
         for (Space *spp : {&ts->cg, &ts->bicg, &ts->amg, &ts->seg.sp}) {
             Space &sp = *spp;
-            for (void *p : {sp.vec, sp.parts, sp.recs, sp.aux, sp.tols, sp.tailDev})
+            for (void *p : {sp.vec, sp.parts, sp.recs, sp.aux, sp.tols, sp.tailDev, sp.link})
                 if (p) (void)hipFree(p);
             if (sp.tailHost) (void)hipHostFree(sp.tailHost);
             if (sp.snap) (void)hipHostFree(sp.snap);

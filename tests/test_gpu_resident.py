@@ -1,0 +1,91 @@
+"""The resident CG engine against the oracle where its shapes change: one workgroup up to the rows its
+registers hold (4096 with five entries per row, 3072 with seven), teams of 512-thread workgroups with
+one, two and four rows per thread, more right-hand sides than run at once, rows longer than the
+kernels take (handed to the other engines).
+
+Tolerances: the engine sums in another order than the oracle, so a solve may stop an iteration
+earlier or later; the solutions then differ by what the stopping residual leaves open, which for these
+shifted operators (smallest eigenvalue >= shift) is at most sqrt(n) tol / shift in the 2-norm."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+SHIFT = 0.05
+
+
+def _grid_operator(shape, extra=None):
+    """2d + 1 point operator of a grid with Dirichlet walls, diagonal 2d + SHIFT + noise; ``extra``: pairs of
+    rows coupled besides."""
+    n, d = int(np.prod(shape)), len(shape)
+    idx = np.arange(n).reshape(shape)
+    rows, cols = [np.arange(n)], [np.arange(n)]
+    for ax in range(d):
+        lo, hi = np.moveaxis(idx, ax, 0)[:-1].ravel(), np.moveaxis(idx, ax, 0)[1:].ravel()
+        rows += [lo, hi]
+        cols += [hi, lo]
+    for i, j in extra or []:
+        rows += [np.array([i, j])]
+        cols += [np.array([j, i])]
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    order = np.lexsort((c, r))
+    r, c = r[order], c[order]
+    row = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32)
+    off = np.bincount(r, minlength=n) - 1
+    diag = np.maximum(2 * d, off) + SHIFT + np.random.default_rng(n).uniform(0, 0.5, n)
+    return row, c.astype(np.int32), np.where(r == c, diag[r], -1.0)
+
+
+def _check(row, col, val, nrhs, dtype, **opts):
+    import phipict_amd as pa
+
+    n = row.size - 1
+    f64 = dtype == np.float64
+    tol = 1e-9 if f64 else 1e-4
+    b = np.random.default_rng(7).standard_normal(nrhs * n).astype(dtype)
+    x0 = (0.1 * np.random.default_rng(8).standard_normal(nrhs * n)).astype(dtype)
+    tdt = torch.float64 if f64 else torch.float32
+    A = pa.CSRmatrix(torch.as_tensor(val, dtype=tdt, device=DEV), torch.as_tensor(col, device=DEV),
+                     torch.as_tensor(row, device=DEV))
+    x = torch.as_tensor(x0.copy(), device=DEV)
+    infos = pa.SolveLinear(A, torch.as_tensor(b, device=DEV), x, maxIterations=4000, tolerance=tol, **opts)
+    xs = x.cpu().numpy().reshape(nrhs, n)
+    for k in sorted({0, nrhs - 1}):
+        xo = x0[k * n:(k + 1) * n].copy()
+        ref = O.cg(row, col, val.astype(dtype), b[k * n:(k + 1) * n].copy(), xo, tol, maxit=4000,
+                   reset_every=opts.get("residualResetSteps", 0), return_best=opts.get("returnBestResult", False))
+        assert infos[k].converged and ref.converged
+        assert abs(infos[k].usedIterations - ref.used_iterations) <= (1 if f64 else 4)
+        bound = 2 * np.sqrt(n) * tol / SHIFT + np.finfo(dtype).eps * 64 * np.linalg.norm(xo)
+        assert np.linalg.norm(xs[k].astype(np.float64) - xo.astype(np.float64)) <= bound, (k, infos[k], ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("shape,nrhs", [
+    ((3, 1), 1), ((63, 65), 2), ((64, 64), 1), ((17, 241), 1),  # one workgroup to its last row, then a team
+    ((12, 16, 16), 1), ((7, 439), 3),                           # 3072 and 3073 rows
+    ((512, 256), 1), ((331, 396), 1),                           # 131072 rows on 256 workgroups, then two rows a thread
+    ((40, 50, 60), 2), ((71, 60, 62), 1),                       # two teams at once; 264120 rows: four rows a thread
+    ((120, 150), 40),                                           # more teams than run at once
+])
+def test_resident_cg_matches_oracle(shape, nrhs, dtype):
+    print(f"[resident] {shape} x {nrhs} {np.dtype(dtype).name}", flush=True)
+    _check(*_grid_operator(shape), nrhs, dtype)
+
+
+@pytest.mark.parametrize("opts", [dict(residualResetSteps=5), dict(returnBestResult=True)], ids=["reset", "best"])
+@pytest.mark.parametrize("shape", [(30, 41), (20, 31, 33)], ids=["workgroup", "team"])
+def test_resident_cg_options(shape, opts):
+    _check(*_grid_operator(shape), 2, np.float64, **opts)
+
+
+@pytest.mark.parametrize("n", [2000, 9000])
+def test_rows_beyond_the_kernels_take_another_engine(n):
+    """One row of 13 entries among rows of five: no rows dropped."""
+    _check(*_grid_operator((n // 50, 50), extra=[(0, n - 1 - 7 * k) for k in range(10)]), 1, np.float64)
