@@ -206,8 +206,8 @@ __device__ __forceinline__ Share share_of(const ResArgs<T> &a, Team &tm, int row
     tm.wgs = a.wgs;
     if (a.P.base) {
         s.piece = a.P.wgPiece[blockIdx.x];
-        tm.wg0 = a.P.wgOff[s.piece];
-        tm.G = a.P.wgOff[s.piece + 1] - tm.wg0;
+        tm.wg0 = a.P.wg0[s.piece];
+        tm.G = a.P.G[s.piece];
         s.n = a.P.len[s.piece];
         s.vbase = a.P.base[s.piece];
         s.mrow = a.P.mrow[s.piece];

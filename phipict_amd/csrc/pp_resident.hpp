@@ -12,10 +12,10 @@ constexpr int RES_LOCAL_WG = 1024; // threads at most of a one-workgroup team
 constexpr int RES_TOLS = 8;        // tolerances passed by value
 
 // Pieces of a segmented solve: piece k has len[k] rows at vector offset base[k], its matrix rows
-// start at mrow[k]; workgroup w works on piece wgPiece[w], whose workgroups are
-// wgOff[k] .. wgOff[k + 1] - 1. All null for a plain solve.
+// start at mrow[k]; workgroup w of the launch works on piece wgPiece[w], whose workgroups are
+// wg0[k] .. wg0[k] + G[k] - 1. All null for a plain solve.
 struct ResPieces {
-    const int32_t *base, *len, *mrow, *wgPiece, *wgOff;
+    const int32_t *base, *len, *mrow, *wg0, *G, *wgPiece;
 };
 
 template <typename T>

@@ -1619,6 +1619,30 @@ static int resident_link(Space &sp, size_t words, uint32_t tags, hipStream_t s, 
 }
 
 constexpr int RES_MAXIT = 1 << 26; // above it the tags of one solve could wrap
+// Exchanges of one launch at most: two sums per iteration, two more per residual replacement.
+static uint32_t resident_tags(int maxit) { return (uint32_t)(4 * ((int64_t)maxit + 4)); }
+
+// Where a resident solve of B right-hand sides leaves its records, then (in the second record copy's
+// place) a word per team and one for failures, told from older contents by this solve's value.
+template <typename T>
+static void resident_status(Space &sp, int B, ResArgs<T> *a) {
+    a->recs = recs_a(sp);
+    a->status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
+    a->failed = a->status + B;
+    a->done = 0xC0DE0000u + (++sp.solves & 0xffffu);
+}
+
+// All of it back in one copy; *ran: every team finished.
+template <typename T>
+static int resident_results(Space &sp, int B, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran) {
+    PP_HIP(hipMemcpyAsync(sp.snap, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 1), hipMemcpyDeviceToHost, s));
+    PP_HIP(hipStreamSynchronize(s));
+    *recs = reinterpret_cast<const SolveRec *>(sp.snap);
+    const unsigned *st = reinterpret_cast<const unsigned *>(sp.snap + sizeof(SolveRec) * B);
+    *ran = st[B] != a.done;
+    for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
+    return PP_OK;
+}
 
 // *ran: the engine finished the solve (false: run another engine; x holds a start guess).
 template <typename T>
@@ -1646,8 +1670,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
     a.tolsDev = ntols > RES_TOLS ? (const double *)sp.tols : nullptr;
     const int maxWgs = plan.perLaunch * plan.G;
     const size_t zWords = plan.local ? 0 : 2 * a.vecLen * (sizeof(T) / 4), slotWords = plan.local ? 0 : (size_t)2 * 3 * maxWgs * 2;
-    // exchanges of one launch at most: two sums per iteration, two more words per residual replacement
-    const uint32_t tags = (uint32_t)(4 * ((int64_t)maxit + 4));
+    const uint32_t tags = resident_tags(maxit);
     const int launches = (B + plan.perLaunch - 1) / plan.perLaunch;
     if (!plan.local && (uint64_t)tags * launches > (1u << 31)) return PP_OK;
     std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
@@ -1659,12 +1682,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
         a.slots = a.zbuf + zWords;
         a.tag = tag;
     }
-    // the records, then (in the second copy's place) a word per team and one for failures, come
-    // back in one copy; the words of this solve are told from older contents by their value
-    a.recs = recs_a(sp);
-    a.status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
-    a.failed = a.status + B;
-    a.done = 0xC0DE0000u + (++sp.solves & 0xffffu);
+    resident_status(sp, B, &a);
     for (int t0 = 0; t0 < B; t0 += plan.perLaunch) {
         const int teams = std::min(plan.perLaunch, B - t0);
         a.team0 = t0;
@@ -1677,14 +1695,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
         a.tag += tags;
         sp.linkTag += plan.local ? 0 : tags;
     }
-    char *host = sp.snap;
-    PP_HIP(hipMemcpyAsync(host, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 1), hipMemcpyDeviceToHost, s));
-    PP_HIP(hipStreamSynchronize(s));
-    *recs = reinterpret_cast<const SolveRec *>(host);
-    const unsigned *st = reinterpret_cast<const unsigned *>(host + sizeof(SolveRec) * B);
-    *ran = st[B] != a.done;
-    for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
-    return PP_OK;
+    return resident_results(sp, B, a, s, recs, ran);
 }
 
 // ---------------- small systems ----------------
@@ -2419,6 +2430,146 @@ static SegLayout seg_layout(const int32_t *segRows, int S, int ncomp, int N, int
 }
 
 
+// Layout upload through a pinned staging copy (rewritten only after a solve's final wait).
+static int upload_layout(SegSpace &sg, const std::vector<int32_t> &host, hipStream_t s) {
+    const size_t bytes = sizeof(int32_t) * host.size();
+    if (sg.layoutHostCap < bytes) {
+        if (sg.layoutHost) (void)hipHostFree(sg.layoutHost);
+        sg.layoutHost = nullptr;
+        sg.layoutHostCap = 0;
+        PP_HIP(hipHostMalloc((void **)&sg.layoutHost, bytes, hipHostMallocDefault));
+        sg.layoutHostCap = bytes;
+    }
+    if (int e = grow((void **)&sg.layoutDev, &sg.layoutCap, bytes)) return e;
+    std::memcpy(sg.layoutHost, host.data(), bytes);
+    PP_HIP(hipMemcpyAsync(sg.layoutDev, sg.layoutHost, bytes, hipMemcpyHostToDevice, s));
+    return PP_OK;
+}
+
+// ---------------- segmented solves on the resident engine ----------------
+// The pieces, longest first, packed into launches of at most one workgroup per CU with R rows per
+// thread; pieces left over that one workgroup holds run together in a last launch of
+// one-workgroup teams (`local` of them). Chosen among R = 1, 2, 4 by the time of the launches, each its
+// longest piece's iterations (about the root of its rows) times the time of one (measured at
+// 8 k - 31 k rows, us): fewer rows per thread iterate faster and need more launches.
+struct SegPack {
+    int R = 0, localR = 0, launches = 0;          // launches of teams
+    double cost = 0.0;
+    std::vector<int32_t> wg0, G, wgPiece, wgFirst; // per piece; per workgroup; per launch, its first workgroup
+};
+
+static SegPack seg_pack(const std::vector<int32_t> &len, int ew, int cus) {
+    const int K = (int)len.size(), localRows = resident_local_rows(ew);
+    std::vector<int> order(K);
+    for (int k = 0; k < K; ++k) order[k] = k;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return len[a] > len[b]; });
+    SegPack best;
+    for (int R : {1, 2, 4}) {
+        const double us = R == 1 ? 4.8 : (R == 2 ? 5.0 : (ew == 5 ? 6.8 : 10.0));
+        SegPack p;
+        p.R = R;
+        p.wg0.assign(K, 0);
+        p.G.assign(K, 1);
+        int at = 0;
+        bool fits = true;
+        while (at < K && fits && (len[order[at]] > localRows || p.launches == 0)) {
+            if (p.launches == 0 && len[order[0]] <= localRows) break; // one workgroup holds every piece
+            p.wgFirst.push_back((int)p.wgPiece.size());
+            p.cost += us * std::sqrt(double(len[order[at]]));
+            int used = 0;
+            while (at < K) {
+                const int k = order[at], G = (len[k] + RES_WG * R - 1) / (RES_WG * R);
+                if (used + G > cus) break;
+                p.wg0[k] = used;
+                p.G[k] = G;
+                p.wgPiece.insert(p.wgPiece.end(), G, k);
+                used += G;
+                ++at;
+            }
+            fits = used > 0;
+            ++p.launches;
+        }
+        if (!fits) continue;
+        p.wgFirst.push_back((int)p.wgPiece.size());
+        if (at < K) {
+            p.localR = (len[order[at]] + RES_LOCAL_WG - 1) / RES_LOCAL_WG;
+            p.cost += (1.2 + 0.45 * p.localR) * std::sqrt(double(len[order[at]]));
+            for (int j = 0; at < K; ++at, ++j) {
+                p.wg0[order[at]] = j;
+                p.wgPiece.push_back(order[at]);
+            }
+        }
+        if (best.R == 0 || p.cost < best.cost) best = p;
+    }
+    return best;
+}
+
+template <typename T>
+static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows, int S, int ncomp, const T *b, T *x,
+                              int maxit, const double *tols, int ntols, int project, hipStream_t s, pp_solve_result *res,
+                              bool *ran) {
+    *ran = false;
+    const int ew = resident_width(A, nnz), N = A.n, K = S * ncomp;
+    if (!ew || maxit > RES_MAXIT) return PP_OK;
+    std::vector<int32_t> base(K), len(K), mrow(K);
+    for (int k = 0; k < K; ++k) {
+        const int c = k / S, p = k % S;
+        base[k] = c * N + segRows[p];
+        len[k] = segRows[p + 1] - segRows[p];
+        mrow[k] = segRows[p];
+    }
+    const SegPack pack = seg_pack(len, ew, std::min(cu_count(), RES_WG));
+    if (!pack.R) return PP_OK;
+    const uint32_t tags = resident_tags(maxit);
+    if ((uint64_t)tags * std::max(1, pack.launches) > (1u << 31)) return PP_OK;
+    SegSpace &sg = my_spaces().seg;
+    Space &sp = sg.sp;
+    if (int e = prepare(sp, 256, 8, K, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
+    // the layout: base len mrow wg0 G [K], wgPiece, through a pinned staging copy (rewritten only after
+    // this solve's final wait)
+    std::vector<int32_t> host;
+    for (const std::vector<int32_t> &v : {base, len, mrow, pack.wg0, pack.G, pack.wgPiece}) host.insert(host.end(), v.begin(), v.end());
+    if (int e = upload_layout(sg, host, s)) return e;
+    const int32_t *ld = sg.layoutDev;
+    ResArgs<T> a{};
+    a.A = A;
+    a.b = b; a.x = x;
+    a.vecLen = (size_t)ncomp * N;
+    a.maxit = maxit; a.project = project; a.zeroStops = 1;
+    a.ntols = ntols > RES_TOLS ? 1 : ntols;
+    for (int k = 0; k < a.ntols; ++k) a.tols[k] = tols[k];
+    a.tolsDev = ntols > RES_TOLS ? (const double *)sp.tols : nullptr;
+    std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
+    if (pack.launches) {
+        alone.lock();
+        const size_t zWords = 2 * a.vecLen * (sizeof(T) / 4);
+        uint32_t tag = 0;
+        if (int e = resident_link(sp, zWords + (size_t)2 * 3 * RES_WG * 2, tags * (uint32_t)pack.launches, s, &tag)) return e;
+        a.zbuf = reinterpret_cast<unsigned long long *>(sp.link);
+        a.slots = a.zbuf + zWords;
+        a.tag = tag;
+    }
+    resident_status(sp, K, &a);
+    for (int l = 0; l < pack.launches + (pack.localR ? 1 : 0); ++l) {
+        const bool local = l == pack.launches;
+        a.wgs = (local ? (int)pack.wgPiece.size() : pack.wgFirst[l + 1]) - pack.wgFirst[l];
+        a.P = ResPieces{ld, ld + K, ld + 2 * K, ld + 3 * K, ld + 4 * K, ld + 5 * K + pack.wgFirst[l]};
+        int e = PP_OK;
+        PP_TIMED(PP_K_CG_SMALL, N, s,
+                 e = launch_resident_cg<T>(a, ew, local ? pack.localR : pack.R, local ? RES_LOCAL_WG : RES_WG, local, s));
+        if (e) return e;
+        a.tag += tags;
+        if (!local) sp.linkTag += tags;
+    }
+    const SolveRec *recs = nullptr;
+    if (int e = resident_results(sp, K, a, s, &recs, ran)) return e;
+    if (!*ran) return PP_OK;
+    report(recs, K, 0, res);
+    for (int k = 0; k < K; ++k)
+        if (recs[k].zero) res[k] = pp_solve_result{0.0, 0, 1, 1, F_MET};
+    return PP_OK;
+}
+
 template <typename T>
 static int seg_solve(const Csr<T> &A, const int32_t *segRows, int S, int ncomp, const T *b, T *x, int maxit,
                      const double *tols, int ntols, int useBicg, int project, int tileRows, hipStream_t s,
@@ -2432,17 +2583,7 @@ static int seg_solve(const Csr<T> &A, const int32_t *segRows, int S, int ncomp, 
     const int nvec = useBicg ? 5 : 5;
     const size_t partDoubles = (size_t)Tt * (useBicg ? (3 + 1 + 3) : (1 + 3 + 1));
     if (int e = prepare(sp, sizeof(T) * nvec * len, partDoubles, K, tols, ntols, s)) return e;
-    // layout upload through a pinned staging copy (rewritten only after this solve's final wait)
-    const size_t lbytes = sizeof(int32_t) * L.host.size();
-    if (g_seg.layoutHostCap < lbytes) {
-        if (g_seg.layoutHost) (void)hipHostFree(g_seg.layoutHost);
-        g_seg.layoutHost = nullptr;
-        PP_HIP(hipHostMalloc((void **)&g_seg.layoutHost, lbytes, hipHostMallocDefault));
-        g_seg.layoutHostCap = lbytes;
-    }
-    if (int e = grow((void **)&g_seg.layoutDev, &g_seg.layoutCap, lbytes)) return e;
-    std::memcpy(g_seg.layoutHost, L.host.data(), lbytes);
-    PP_HIP(hipMemcpyAsync(g_seg.layoutDev, g_seg.layoutHost, lbytes, hipMemcpyHostToDevice, s));
+    if (int e = upload_layout(g_seg, L.host, s)) return e;
     const int32_t *ld = g_seg.layoutDev;
     seg::Pieces P{ld, ld + K, ld + 2 * K, ld + 4 * K + 1, ld + 4 * K + 1 + Tt, ld + 3 * K, K, Tt, tileRows, N};
     // everything the iteration kernels are given, for the captured chunks
@@ -2690,6 +2831,14 @@ int pp_solve_segmented(const pp_csr *A, const int32_t *seg_rows, int32_t nseg, i
     
     PP_DISPATCH(dtype, {
         const Csr<T> C = csr_view<T>(A, 1);
+        if (!use_bicg) {
+            bool ran = false;
+            if (int e = resident_segmented<T>(C, A->nnz, seg_rows, nseg, ncomp, reinterpret_cast<const T *>(rhs),
+                                              reinterpret_cast<T *>(x), maxit, tols, ntols, project, as_stream(stream),
+                                              results, &ran))
+                return e;
+            if (ran) return PP_OK;
+        }
         return seg_solve<T>(C, seg_rows, nseg, ncomp, reinterpret_cast<const T *>(rhs), reinterpret_cast<T *>(x), maxit,
                             tols, ntols, use_bicg, project, tile_rows, as_stream(stream), results);
     });

@@ -89,3 +89,40 @@ def test_resident_cg_options(shape, opts):
 def test_rows_beyond_the_kernels_take_another_engine(n):
     """One row of 13 entries among rows of five: no rows dropped."""
     _check(*_grid_operator((n // 50, 50), extra=[(0, n - 1 - 7 * k) for k in range(10)]), 1, np.float64)
+
+
+@pytest.mark.parametrize("shapes,ncomp", [
+    ([(9, 7), (64, 64), (30, 2)], 2),                     # one workgroup each
+    ([(65, 64), (20, 11), (300, 220), (3, 3)], 1),        # teams, the small ones beside them
+    ([(420, 400)] * 3 + [(200, 150), (31, 17)], 1),       # 504 k rows: several launches
+    ([(14, 15, 16), (33, 31, 30), (8, 9, 10)], 2),        # seven entries per row
+], ids=["local", "mixed", "launches", "3d"])
+def test_resident_segmented_cg_matches_oracle(shapes, ncomp):
+    import phipict_amd as pa
+
+    parts = [_grid_operator(s) for s in shapes]
+    segs = np.concatenate([[0], np.cumsum([p[0].size - 1 for p in parts])])
+    row = np.concatenate([[0]] + [p[0][1:] + off for p, off in
+                                  zip(parts, np.concatenate([[0], np.cumsum([p[1].size for p in parts])]))]).astype(np.int32)
+    col = np.concatenate([p[1] + o for p, o in zip(parts, segs)]).astype(np.int32)
+    val = np.concatenate([p[2] for p in parts])
+    n, S, tol = int(segs[-1]), len(shapes), 1e-9
+    rng = np.random.default_rng(11)
+    b, x0 = rng.standard_normal((ncomp, n)), 0.1 * rng.standard_normal((ncomp, n))
+    b[0, segs[1]:segs[2]] = 0.0  # a zero right-hand side: x = 0, no iterations
+    A = pa.CSRmatrix(*(torch.as_tensor(a, device=DEV) for a in (val, col, row)))
+    x = torch.as_tensor(x0.reshape(-1).copy(), device=DEV)
+    infos = pa.SolveSegmented(A, segs.tolist(), torch.as_tensor(b.reshape(-1), device=DEV), x, maxIterations=4000,
+                              tolerance=tol)
+    xs = x.cpu().numpy().reshape(ncomp, n)
+    for c in range(ncomp):
+        for s in range(S):
+            lo, hi = int(segs[s]), int(segs[s + 1])
+            info = infos[c * S + s]
+            if not b[c, lo:hi].any():
+                assert info.converged and info.usedIterations == 0 and not xs[c, lo:hi].any()
+                continue
+            xo = x0[c, lo:hi].copy()
+            ref = O.cg(*parts[s], b[c, lo:hi].copy(), xo, tol, maxit=4000)
+            assert info.converged and abs(info.usedIterations - ref.used_iterations) <= 1
+            assert np.linalg.norm(xs[c, lo:hi] - xo) <= 2 * np.sqrt(hi - lo) * tol / SHIFT + 1e-14 * np.linalg.norm(xo)
