@@ -142,7 +142,8 @@ typedef struct pp_domain {
     void *scalar_rhs;       /* [batch][C][n] */
     void *scalar_result;    /* [batch][C][n] */
     int32_t advection_scheme; /* PP_ADV_CENTRAL / PP_ADV_LINEAR_UPWIND (Domain::setAdvectionScheme) */
-    int32_t reserved;
+    int32_t unconnected;    /* 1: every face is PERIODIC or FIXED and every block has two or more cells along
+                             * each axis (lets the corner terms skip the walks); 0: not known */
 } pp_domain;
 
 /* The reference's LinearSolverResultInfo (csrc/phipict/solvers/linear_solvers.h:180-185). */

@@ -107,7 +107,7 @@ class DomainDesc(C.Structure):
         ("scalar_rhs", C.c_void_p),
         ("scalar_result", C.c_void_p),
         ("advection_scheme", C.c_int32),
-        ("reserved", C.c_int32),
+        ("unconnected", C.c_int32),
     ]
 
 

@@ -158,6 +158,13 @@ __device__ __forceinline__ int asm_tile() {
     int p[3];                                                                  \
     unflat(f, b.size, p);
 
+// The template argument NO of the kernels with corner terms: 0 without them, 2 with them for any
+// cell, 1 with them where no cell touches a block connection (the domain says so), without the
+// walks: in one kernel the walks' registers and code burden the cells that never walk. 393 k skewed
+// cells, FP64: advection matrix 109 us with the walks in the kernel, 63 us without (walking 213 us);
+// pressure matrix 80 / 48 (171), momentum right-hand side 74 / 70 (227), divergence 43 / 45 (137).
+static int corner_mode(const pp_domain *dom, int flags) { return flags == 0 ? 0 : (dom->unconnected ? 1 : 2); }
+
 // CSR pattern: row offsets and ascending neighbour columns of every row (shared by the
 // advection, pressure and potential matrices; row layout of topology.cuh:168-233).
 template <int D>
@@ -208,7 +215,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_csr_pattern(pp_domain dom, int32_
 // matrix of passive-scalar channel sc (forPassiveScalar): the channel's diffusivity and its
 // boundary condition at the prescribed faces. LINEAR_UPWIND puts first-order upwind on the
 // faces whose far-upwind cell lies in the block (advection.cu:129-140), CENTRAL elsewhere.
-template <typename T, int D, bool NO>
+template <typename T, int D, int NO>
 __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, int sc, int flags) {
     CELL_PROLOGUE
     const T dt = reinterpret_cast<const T *>(dom.time_step)[env];
@@ -225,6 +232,12 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, i
     T ap[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) ap[k] = Metric<T, D>::alpha(b, f, k);
+    Near<D> nr;
+    Cross<T, D> cP;
+    if (NO && flags) {
+        nr = near_cell<D>(b, p);
+        cP.load(b, f);
+    }
 #pragma unroll
     for (int bound = 0; bound < 2 * D; ++bound) {
         const int dim = bound >> 1;
@@ -248,7 +261,19 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, i
             const T vc = (ap[dim] * vp + an * vn) * T(0.5);
             diag += vc;
             rv[bound + 1] -= vc;
-            if (NO && flags) {
+            if (NO && flags && (NO == 1 || nr.ok)) {
+                Cross<T, D> cN;
+                cN.load(b, nf);
+                if (sc < 0) {
+                    const CornerData<T, D, NK_VELOCITY_TYPES> cd{dom, blocks, 0, env};
+                    matrix_corner_near<T, D, NK_VELOCITY_TYPES>(cd, bi, nr, p, bound, flags, cP, cN, vp, vn, T(1), false,
+                                                                T(1), diag, rv);
+                } else {
+                    const CornerData<T, D, NK_SCALAR_TYPES> cd{dom, blocks, sc, env};
+                    matrix_corner_near<T, D, NK_SCALAR_TYPES>(cd, bi, nr, p, bound, flags, cP, cN, T(1), T(1), vp, false,
+                                                              T(1), diag, rv);
+                }
+            } else if (NO == 2 && flags) {
                 if (sc < 0) {
                     const CornerData<T, D, NK_VELOCITY_TYPES> cd{dom, blocks, 0, env};
                     matrix_corner_terms<T, D, NK_VELOCITY_TYPES>(cd, bi, p, f, bound, flags, vp, true, nullptr, T(1),
@@ -291,21 +316,21 @@ __device__ T pressure_at(const pp_domain &dom, const pp_block_desc *__restrict__
         const pp_boundary_desc &bd = b.bnd[dim * 2 + (upper ? 1 : 0)];
         if (bd.type == PP_BOUND_FIXED) {
             t[dim] = lower ? 0 : b.size[dim] - 1;
-            return reinterpret_cast<const T *>(b.pressure)[(size_t)env * b.cells + flat3(t, b.size)];
+            return gptr<const T>(b.pressure)[(size_t)env * b.cells + flat3(t, b.size)];
         }
         if (bd.type == PP_BOUND_CONNECTED) {
             int op[3];
             conn_pos(blocks, D, t, dim, bd, lower ? -(pin[dim] + 1) : pin[dim] - b.size[dim], op);
             const pp_block_desc &nb = blocks[bd.conn_block];
-            return reinterpret_cast<const T *>(nb.pressure)[(size_t)env * nb.cells + flat3(op, nb.size)];
+            return gptr<const T>(nb.pressure)[(size_t)env * nb.cells + flat3(op, nb.size)];
         }
         if (bd.type == PP_BOUND_PERIODIC) {
             t[dim] += lower ? b.size[dim] : -b.size[dim];
-            return reinterpret_cast<const T *>(b.pressure)[(size_t)env * b.cells + flat3(t, b.size)];
+            return gptr<const T>(b.pressure)[(size_t)env * b.cells + flat3(t, b.size)];
         }
         return T(0);
     }
-    return reinterpret_cast<const T *>(b.pressure)[(size_t)env * b.cells + flat3(pin, b.size)];
+    return gptr<const T>(b.pressure)[(size_t)env * b.cells + flat3(pin, b.size)];
 }
 
 // getPressureGradient, velocity.cuh:347-382 (FD, transformed with Minv^T)
@@ -372,12 +397,12 @@ __device__ __forceinline__ T boundary_source(const pp_domain &dom, const pp_bloc
 
 // kPISO_build_advection_RHS, advection.cu:799-955 (with LINEAR_UPWIND the deferred correction
 // of the block velocity, lagged to the start of the step)
-template <typename T, int D, bool NO>
+template <typename T, int D, int NO>
 __global__ void __launch_bounds__(ASM_BLOCK) k_advection_rhs(pp_domain dom, int apply_pg, int flags) {
     CELL_PROLOGUE
     const T dt = reinterpret_cast<const T *>(dom.time_step)[env];
     const T det = Metric<T, D>::det(b, f);
-    const T *vel = reinterpret_cast<const T *>(b.velocity) + (size_t)env * D * b.cells;
+    const T *vel = gptr<const T>(b.velocity) + (size_t)env * D * b.cells;
     const bool deferred = dom.advection_scheme == PP_ADV_LINEAR_UPWIND;
     T fl[2 * D];
     if (deferred) cell_fluxes<T, D, false>(dom, blocks, bi, p, f, nullptr, env, fl);
@@ -388,7 +413,9 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_rhs(pp_domain dom, int 
     T Sv[D];
     if (NO && flags) {
         const CornerData<T, D, NK_VELOCITY> cd{dom, blocks, 0, env};
-        nonortho_rhs<T, D, NK_VELOCITY>(cd, bi, p, f, flags, true, nullptr, Sv);
+        const Near<D> nr = near_cell<D>(b, p);
+        if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_VELOCITY>(cd, bi, nr, p, f, flags, true, nullptr, Sv);
+        else if constexpr (NO == 2) nonortho_rhs<T, D, NK_VELOCITY>(cd, bi, p, f, flags, true, nullptr, Sv);
     }
 #pragma unroll
     for (int dim = 0; dim < D; ++dim) {
@@ -422,13 +449,13 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_rhs(pp_domain dom, int 
 // prescribed faces give the advected face value and the diffusive flux (Dirichlet: the face
 // value with the ghost-cell coefficient 2 alpha; Neumann: the cell value advected and the
 // prescribed normal gradient times the face area); with LINEAR_UPWIND the deferred correction
-template <typename T, int D, bool NO>
+template <typename T, int D, int NO>
 __global__ void __launch_bounds__(ASM_BLOCK) k_scalar_rhs(pp_domain dom, int flags) {
     CELL_PROLOGUE
     const int C = dom.scalar_channels;
     const T dt = reinterpret_cast<const T *>(dom.time_step)[env];
     const T det = Metric<T, D>::det(b, f);
-    const T *phi = reinterpret_cast<const T *>(b.scalar) + (size_t)env * C * b.cells;
+    const T *phi = gptr<const T>(b.scalar) + (size_t)env * C * b.cells;
     T *rhs = reinterpret_cast<T *>(dom.scalar_rhs) + (size_t)env * C * dom.num_cells;
     const bool deferred = dom.advection_scheme == PP_ADV_LINEAR_UPWIND;
     T fl[2 * D];
@@ -464,8 +491,10 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_scalar_rhs(pp_domain dom, int fla
         if (deferred) deferred_correction<T, D>(b, p, fl, phi + (size_t)ch * b.cells, t);
         if (NO && flags) {
             const CornerData<T, D, NK_SCALAR> cd{dom, blocks, ch, env};
+            const Near<D> nr = near_cell<D>(b, p);
             T S[1];
-            nonortho_rhs<T, D, NK_SCALAR>(cd, bi, p, f, flags, false, nullptr, S);
+            if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_SCALAR>(cd, bi, nr, p, f, flags, false, nullptr, S);
+            else if constexpr (NO == 2) nonortho_rhs<T, D, NK_SCALAR>(cd, bi, p, f, flags, false, nullptr, S);
             t -= S[0] * scalar_visc<T>(dom, ch);
         }
         rhs[(size_t)ch * dom.num_cells + g] = t / det;
@@ -473,7 +502,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_scalar_rhs(pp_domain dom, int fla
 }
 
 // PISO_build_pressure_matrix, pressure.cu:25-193 (useFaceTransform = false)
-template <typename T, int D, bool NO>
+template <typename T, int D, int NO>
 __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_matrix(pp_domain dom, int flags) {
     CELL_PROLOGUE
     const T *A = reinterpret_cast<const T *>(dom.A) + (size_t)env * dom.num_cells;
@@ -486,6 +515,12 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_matrix(pp_domain dom, in
     for (int k = 0; k < D; ++k) ap[k] = Metric<T, D>::alpha(b, f, k);
     const T raP = T(1.0) / A[g];
     idx[0] = g;
+    Near<D> nr;
+    Cross<T, D> cP;
+    if (NO && flags) {
+        nr = near_cell<D>(b, p);
+        cP.load(b, f);
+    }
 #pragma unroll
     for (int bound = 0; bound < 2 * D; ++bound) {
         const int dim = bound >> 1;
@@ -503,8 +538,15 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_matrix(pp_domain dom, in
             idx[bound + 1] = ng;
             if (NO && flags) {
                 const CornerData<T, D, NK_FIXED_ONLY> cd{dom, blocks, 0, env};
-                matrix_corner_terms<T, D, NK_FIXED_ONLY>(cd, bi, p, f, bound, flags, raP, false, A, T(1), true, T(-1),
-                                                         rv[0], rv);
+                if (NO == 1 || nr.ok) {
+                    Cross<T, D> cN;
+                    cN.load(b, nf);
+                    matrix_corner_near<T, D, NK_FIXED_ONLY>(cd, bi, nr, p, bound, flags, cP, cN, raP, raN, T(1), true, T(-1),
+                                                            rv[0], rv);
+                } else if constexpr (NO == 2) {
+                    matrix_corner_terms<T, D, NK_FIXED_ONLY>(cd, bi, p, f, bound, flags, raP, false, A, T(1), true, T(-1),
+                                                             rv[0], rv);
+                }
             }
         } else {
             idx[bound + 1] = -1;
@@ -525,7 +567,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_rhs(pp_domain dom) {
     const T rDiag = 1 / reinterpret_cast<const T *>(dom.A)[(size_t)env * dom.num_cells + g];
     const T det = Metric<T, D>::det(b, f);
     const T *vres = reinterpret_cast<const T *>(dom.velocity_result) + (size_t)env * D * dom.num_cells;
-    const T *vel = reinterpret_cast<const T *>(b.velocity) + (size_t)env * D * b.cells;
+    const T *vel = gptr<const T>(b.velocity) + (size_t)env * D * b.cells;
     T *prhs = reinterpret_cast<T *>(dom.pressure_rhs) + (size_t)env * D * dom.num_cells;
     // off-diagonal part of C times the predicted velocity, all components in one pass over the row
     T Hs[D];
@@ -567,7 +609,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_rhs(pp_domain dom) {
 }
 
 // k_computePressureRHSdivergenceFromFlux, pressure.cu:755-803 (useFaceTransform = false)
-template <typename T, int D, bool NO>
+template <typename T, int D, int NO>
 // With the flags' right-hand-side bits it also adds the pressure's explicit corner terms
 // (k_pressureRHSaddNonOrthoComponents, pressure.cu:838-860).
 __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_div(pp_domain dom, int time_step_norm, int flags) {
@@ -581,9 +623,11 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_div(pp_domain dom, int t
     if (time_step_norm) dv /= reinterpret_cast<const T *>(dom.time_step)[env];
     if (NO && (flags & (NO_DIRECT_RHS | NO_DIAGONAL_RHS))) {
         const CornerData<T, D, NK_PRESSURE> cd{dom, blocks, 0, env};
+        const T *A = reinterpret_cast<const T *>(dom.A) + (size_t)env * dom.num_cells;
+        const Near<D> nr = near_cell<D>(b, p);
         T S[1];
-        nonortho_rhs<T, D, NK_PRESSURE>(cd, bi, p, f, flags, false,
-                                        reinterpret_cast<const T *>(dom.A) + (size_t)env * dom.num_cells, S);
+        if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_PRESSURE>(cd, bi, nr, p, f, flags, false, A, S);
+        else if constexpr (NO == 2) nonortho_rhs<T, D, NK_PRESSURE>(cd, bi, p, f, flags, false, A, S);
         dv += S[0];
     }
     reinterpret_cast<T *>(dom.pressure_rhs_div)[(size_t)env * dom.num_cells + g] = dv;
@@ -818,7 +862,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_copy_result(pp_domain dom, int fi
     if (f >= b.cells) return;
     const int g = b.global_offset + f;
     const int env = blockIdx.y;
-    T *bf = reinterpret_cast<T *>(field == 0 ? b.velocity : (field == 1 ? b.pressure : (field == 2 ? b.epot : b.scalar)));
+    T *bf = gptr<T>(field == 0 ? b.velocity : (field == 1 ? b.pressure : (field == 2 ? b.epot : b.scalar)));
     if (!bf) return;
     for (int c = 0; c < ch; ++c) {
         const size_t fo = ((size_t)env * ch + c) * dom.num_cells + g;
@@ -1625,7 +1669,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_max_velocity(pp_domain dom, int f
         if (withBounds && b.bnd[f].type == PP_BOUND_FIXED) units += cells / b.size[f >> 1];
     }
     faceStart[2 * D] = units;
-    const T *vel = reinterpret_cast<const T *>(b.velocity) + (size_t)env * D * cells;
+    const T *vel = gptr<const T>(b.velocity) + (size_t)env * D * cells;
     const bool cellTransform = computational && b.has_transform;
     T m = 0;
     for (int u = tile * ASM_BLOCK + threadIdx.x; u < units; u += wpb * ASM_BLOCK) {
@@ -1643,7 +1687,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_max_velocity(pp_domain dom, int f
             const int ff = u - faceStart[f];
             const int fc = faceStart[f + 1] - faceStart[f];
             const int vb = fb.vel_batched ? env : 0;
-            const T *fv = reinterpret_cast<const T *>(fb.vel);
+            const T *fv = gptr<const T>(fb.vel);
 #pragma unroll
             for (int c = 0; c < D; ++c)
                 v[c] = fb.vel_static ? fv[(size_t)vb * D + c] : fv[((size_t)vb * D + c) * fc + ff];
@@ -1756,7 +1800,7 @@ int pp_setup_advection_matrix(const pp_domain *dom, int32_t non_ortho_flags, voi
     const int flags = matrix_flags(non_ortho_flags);
     PP_CHECK_ARG(dom->C.val && dom->C.row && dom->A && dom->time_step, "C, A and time_step must be set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_ADVECTION_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((flags ? k_advection_matrix<T, D, true> : k_advection_matrix<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, -1, flags))));
+        PP_TIMED(PP_K_ADVECTION_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_matrix<T, D, 1> : k_advection_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, -1, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1768,7 +1812,7 @@ int pp_setup_advection_matrix_scalar(const pp_domain *dom, int32_t non_ortho_fla
     PP_CHECK_ARG(channel >= 0 && channel < dom->scalar_channels, "passive scalar channel out of range");
     PP_CHECK_ARG(dom->scalar_visc_count == 0 || dom->scalar_viscosity, "scalar viscosity not set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        hipLaunchKernelGGL((flags ? k_advection_matrix<T, D, true> : k_advection_matrix<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, (int)channel, flags)));
+        hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_matrix<T, D, 1> : k_advection_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, (int)channel, flags)));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1780,7 +1824,7 @@ int pp_setup_advection_scalar(const pp_domain *dom, int32_t non_ortho_flags, voi
     PP_CHECK_ARG(!flags || dom->scalar_result, "the non-orthogonal terms read scalar_result");
     PP_CHECK_ARG(dom->scalar_visc_count == 0 || dom->scalar_viscosity, "scalar viscosity not set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        hipLaunchKernelGGL((flags ? k_scalar_rhs<T, D, true> : k_scalar_rhs<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags)));
+        hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_scalar_rhs<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_scalar_rhs<T, D, 1> : k_scalar_rhs<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags)));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1791,7 +1835,7 @@ int pp_setup_advection_velocity(const pp_domain *dom, int32_t non_ortho_flags, i
     PP_CHECK_ARG(dom->velocity_rhs && dom->time_step, "velocity_rhs and time_step must be set");
     PP_CHECK_ARG(!flags || dom->velocity_result, "the non-orthogonal terms read velocity_result");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_ADVECTION_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((flags ? k_advection_rhs<T, D, true> : k_advection_rhs<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_ADVECTION_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_rhs<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_rhs<T, D, 1> : k_advection_rhs<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)apply_pressure_gradient, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
@@ -1802,7 +1846,7 @@ int pp_setup_pressure_matrix(const pp_domain *dom, int32_t non_ortho_flags, void
     const int flags = matrix_flags(non_ortho_flags);
     PP_CHECK_ARG(dom->P.val && dom->P.row && dom->A, "P and A must be set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_PRESSURE_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((flags ? k_pressure_matrix<T, D, true> : k_pressure_matrix<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags))));
+        PP_TIMED(PP_K_PRESSURE_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_matrix<T, D, 1> : k_pressure_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1814,7 +1858,7 @@ int pp_setup_pressure_rhs(const pp_domain *dom, int32_t non_ortho_flags, int32_t
     PP_CHECK_ARG(!flags || (dom->pressure_result && dom->A), "the non-orthogonal terms read pressure_result and A");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
         PP_TIMED(PP_K_PRESSURE_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((k_pressure_rhs<T, D>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom));
-        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((flags ? k_pressure_div<T, D, true> : k_pressure_div<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_div<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_div<T, D, 1> : k_pressure_div<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)time_step_norm, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
@@ -1826,7 +1870,7 @@ int pp_setup_pressure_rhs_div(const pp_domain *dom, int32_t non_ortho_flags, int
     PP_CHECK_ARG(dom->pressure_rhs && dom->pressure_rhs_div, "pressure fields must be set");
     PP_CHECK_ARG(!flags || (dom->pressure_result && dom->A), "the non-orthogonal terms read pressure_result and A");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((flags ? k_pressure_div<T, D, true> : k_pressure_div<T, D, false>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_div<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_div<T, D, 1> : k_pressure_div<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)time_step_norm, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;

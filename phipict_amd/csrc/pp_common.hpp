@@ -70,6 +70,14 @@ template <typename T> __device__ __forceinline__ T dsqrt(T x);
 template <> __device__ __forceinline__ float dsqrt<float>(float x) { return sqrtf(x); }
 template <> __device__ __forceinline__ double dsqrt<double>(double x) { return sqrt(x); }
 
+// A device address of a descriptor as a pointer the compiler knows to be global memory: through a plain
+// cast every access is a flat one, which counts against scalar and LDS loads as well, so that each
+// wait for a descriptor field also waits for all field data in flight.
+template <typename P>
+__device__ __forceinline__ P *gptr(uint64_t address) {
+    return (P *)(__attribute__((address_space(1))) P *)address;
+}
+
 struct Pos { int a[3]; };
 
 __device__ __forceinline__ int flat3(const int *p, const int32_t *s) { return p[0] + s[0] * (p[1] + s[1] * p[2]); }
@@ -171,10 +179,10 @@ template <typename T, int D>
 struct Metric {
     static constexpr int TS = 2 * D * D + 1;
     __device__ static __forceinline__ TView<T> at(const pp_block_desc &b, int f) {
-        return TView<T>{reinterpret_cast<const T *>(b.transform) + f, b.cells};
+        return TView<T>{gptr<const T>(b.transform) + f, b.cells};
     }
     __device__ static __forceinline__ TView<T> face(const pp_boundary_desc &fb, int ff) {
-        return TView<T>{reinterpret_cast<const T *>(fb.transform) + (size_t)ff * TS, 1};
+        return TView<T>{gptr<const T>(fb.transform) + (size_t)ff * TS, 1};
     }
     __device__ static __forceinline__ T det(const pp_block_desc &b, int f) {
         if (!b.has_transform) return T(1);
@@ -229,7 +237,7 @@ struct Metric {
 template <typename T>
 __device__ __forceinline__ T visc_at(const pp_domain &dom, const pp_block_desc &b, int f) {
     if (b.visc_mode == 0) return T(dom.viscosity);
-    const T *v = reinterpret_cast<const T *>(b.viscosity);
+    const T *v = gptr<const T>(b.viscosity);
     return b.visc_mode == 1 ? v[0] : v[f];
 }
 
@@ -243,13 +251,13 @@ __device__ __forceinline__ T scalar_visc(const pp_domain &dom, int ch) {
 }
 // passive-scalar condition of a fixed face for channel ch (Dirichlet when no types are given)
 __device__ __forceinline__ bool scalar_neumann(const pp_boundary_desc &fb, int ch) {
-    return fb.scalar_types && reinterpret_cast<const int8_t *>(fb.scalar_types)[ch] == PP_BC_NEUMANN;
+    return fb.scalar_types && gptr<const int8_t>(fb.scalar_types)[ch] == PP_BC_NEUMANN;
 }
 // passive-scalar face data of channel ch at face cell ff (0 when the face has none)
 template <typename T>
 __device__ __forceinline__ T fixed_scalar(const pp_boundary_desc &fb, int C, int fc, int ff, int ch, int env) {
     if (!fb.scalar) return T(0);
-    const T *data = reinterpret_cast<const T *>(fb.scalar);
+    const T *data = gptr<const T>(fb.scalar);
     const int e = fb.scalar_batched ? env : 0;
     if (fb.scalar_static) return data[e * C + ch];
     return data[((size_t)e * C + ch) * fc + ff];
@@ -261,7 +269,7 @@ template <typename T>
 __device__ __forceinline__ T vel_at(const pp_domain &dom, const pp_block_desc &b, int f, int k, const T *glob,
                                     int env) {
     if (glob) return glob[(size_t)k * dom.num_cells + b.global_offset + f];
-    return reinterpret_cast<const T *>(b.velocity)[((size_t)env * dom.dims + k) * b.cells + f];
+    return gptr<const T>(b.velocity)[((size_t)env * dom.dims + k) * b.cells + f];
 }
 
 template <typename T, int D>
@@ -303,7 +311,7 @@ __device__ __forceinline__ void contra_all(const pp_domain &dom, const pp_block_
 // FIXED boundary velocity component k at face cell ff (getFixedBoundaryData, block_data.cuh:123-196)
 template <typename T>
 __device__ __forceinline__ T fixed_vel(const pp_boundary_desc &fb, int d, int fc, int ff, int k, int env) {
-    const T *data = reinterpret_cast<const T *>(fb.vel);
+    const T *data = gptr<const T>(fb.vel);
     const int e = fb.vel_batched ? env : 0;
     if (fb.vel_static) return data[e * d + k];
     return data[((size_t)e * d + k) * fc + ff];
@@ -325,7 +333,7 @@ __device__ __forceinline__ T alpha_fixed(const pp_boundary_desc &fb, int ff, int
 template <typename T>
 __device__ __forceinline__ T vsource(const pp_domain &dom, const pp_block_desc &b, int f, int k, int env) {
     if (b.vsource_mode == 0) return T(0);
-    const T *s = reinterpret_cast<const T *>(b.vsource);
+    const T *s = gptr<const T>(b.vsource);
     const int e = b.vsource_batched ? env : 0;
     if (b.vsource_mode == 1) return s[e * dom.dims + k];
     return s[((size_t)e * dom.dims + k) * b.cells + f];
@@ -333,14 +341,14 @@ __device__ __forceinline__ T vsource(const pp_domain &dom, const pp_block_desc &
 __device__ __forceinline__ int pot_bc(const pp_block_desc &b, int bound, const int *p) {
     const pp_boundary_desc &fb = b.bnd[bound];
     if (!fb.pot_types) return fb.pot_type;
-    return reinterpret_cast<const int8_t *>(fb.pot_types)[face_flat(p, bound, b)];
+    return gptr<const int8_t>(fb.pot_types)[face_flat(p, bound, b)];
 }
 template <typename T>
 __device__ __forceinline__ T pot_value(const pp_block_desc &b, int bound, const int *p, int env) {
     const pp_boundary_desc &fb = b.bnd[bound];
     if (!fb.pot_values) return T(0);
     const size_t e = fb.pot_values_batched ? (size_t)env * face_cells(b, bound) : 0;
-    return reinterpret_cast<const T *>(fb.pot_values)[e + face_flat(p, bound, b)];
+    return gptr<const T>(fb.pot_values)[e + face_flat(p, bound, b)];
 }
 __device__ __forceinline__ bool is_epot_dirichlet(const pp_block_desc &b, int bound, const int *p) {
     return b.bnd[bound].type == PP_BOUND_FIXED && pot_bc(b, bound, p) == PP_POT_DIRICHLET;

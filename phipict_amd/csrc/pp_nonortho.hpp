@@ -117,9 +117,9 @@ struct CornerData {
     const pp_block_desc *__restrict__ blocks;
     int w;   // scalar channel
     int env;
-    __device__ __forceinline__ void cell(int bi, const P3 &p, T *out) const {
-        const pp_block_desc &b = blocks[bi];
-        const size_t g = (size_t)b.global_offset + flat_p(p, b);
+    __device__ __forceinline__ void cell(int bi, const P3 &p, T *out) const { at(bi, flat_p(p, blocks[bi]), out); }
+    __device__ __forceinline__ void at(int bi, int f, T *out) const {
+        const size_t g = (size_t)blocks[bi].global_offset + f;
         const size_t n = dom.num_cells;
         if (KIND == NK_VELOCITY) {
 #pragma unroll
@@ -454,6 +454,203 @@ __device__ __forceinline__ void nonortho_rhs(const CornerData<T, D, KIND> &cd, i
                 } else {
 #pragma unroll
                     for (int k = 0; k < NC; ++k) tg[k] += T(tfs) * cv.data[k];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < NC; ++k) S[k] -= T(fs) * faceAlpha * tg[k];
+        }
+    }
+}
+
+// ---- the same terms for cells that touch no block connection ----
+// Away from connections the walk around a corner always ends the same way: at the diagonal cell, or at
+// the prescribed face on its tangential side. Its cells are then constant offsets from the cell
+// (the periodic seam wraps), so the terms are plain loads instead of walks: no descriptor of another
+// block and no per-lane block index. The terms are added in the walks' order. The walks above stay for cells at a connection and blocks one cell thick.
+template <int D>
+struct Near {
+    int d[2 * D];     // offset of the neighbour across each face (0 where there is none)
+    bool wall[2 * D]; // the cell's face is a prescribed face
+    bool ok;          // the cell touches no connection
+};
+template <int D>
+__device__ __forceinline__ Near<D> near_cell(const pp_block_desc &b, const int *p) {
+    Near<D> n;
+    n.ok = true;
+    int stride = 1;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const int last = b.size[a] - 1;
+        n.ok = n.ok && last > 0;
+#pragma unroll
+        for (int up = 0; up < 2; ++up) {
+            const int face = 2 * a + up, type = b.bnd[face].type;
+            const bool at = up ? p[a] == last : p[a] == 0;
+            n.wall[face] = at && type == PP_BOUND_FIXED;
+            n.ok = n.ok && !(at && type != PP_BOUND_FIXED && type != PP_BOUND_PERIODIC);
+            const int step = !at ? 1 : (type == PP_BOUND_PERIODIC ? -last : 0);
+            n.d[face] = up ? step * stride : -step * stride;
+        }
+        stride *= b.size[a];
+    }
+    return n;
+}
+
+// The cross coefficients alpha_{c1 c2}, c1 < c2, of a cell.
+template <typename T, int D>
+struct Cross {
+    T v[D == 2 ? 1 : 3];
+    __device__ __forceinline__ T at(int c1, int c2) const { return v[D == 2 ? 0 : c1 + c2 - 1]; }
+    __device__ __forceinline__ void load(const pp_block_desc &b, int f) {
+#pragma unroll
+        for (int k = 0; k < (D == 2 ? 1 : 3); ++k) v[k] = T(0);
+        if (!b.has_transform) return;
+        const TView<T> t = Metric<T, D>::at(b, f);
+        v[0] = lap_coef_t<T, D>(t, 0, 1);
+        if constexpr (D == 3) {
+            v[1] = lap_coef_t<T, D>(t, 0, 2);
+            v[2] = lap_coef_t<T, D>(t, 1, 2);
+        }
+    }
+};
+
+// matrix_corner_terms for face `bound` of such a cell: cP, cN its and the neighbour's cross
+// coefficients, raP, raN their weights.
+template <typename T, int D, int KIND>
+__device__ __forceinline__ void matrix_corner_near(const CornerData<T, D, KIND> &cd, int bi, const Near<D> &nr, const int *p,
+                                                   int bound, int flags, const Cross<T, D> &cP, const Cross<T, D> &cN,
+                                                   T raP, T raN, T vscale, bool always_gradient, T sign, T &diag, T *rv) {
+    const bool nbr = flags & NO_DIRECT_MATRIX, ctr = flags & NO_CENTER_MATRIX;
+    if (!(nbr || ctr)) return;
+    const pp_block_desc &b = cd.blocks[bi];
+    const int dim = bound >> 1;
+    if (is_fixed(b, bound) && (p[dim] == 0 || p[dim] == b.size[dim] - 1)) return;
+#pragma unroll
+    for (int i = 1; i < D; ++i) {
+        const int tAxis = (dim + i) % D;
+        const T alpha = (cP.at(dim, tAxis) * raP + cN.at(dim, tAxis) * raN) * T(0.5) * vscale;
+#pragma unroll
+        for (int tUp = 0; tUp < 2; ++tUp) {
+            const int tFace = tAxis * 2 + tUp;
+            const T c = T(face_sign(bound) * face_sign(tFace)) * alpha * T(0.25);
+            if (!nr.wall[tFace]) {
+                if (ctr) diag -= sign * c;
+                if (nbr) {
+                    rv[bound + 1] -= sign * c;
+                    rv[tFace + 1] -= sign * c;
+                }
+            } else if (always_gradient || cd.neumann(bi, tFace)) {
+                if (ctr) diag -= sign * (3 * c);
+                if (nbr) {
+                    rv[bound + 1] -= sign * (3 * c);
+                    rv[(tFace ^ 1) + 1] += sign * c;
+                }
+            }
+        }
+    }
+}
+
+// nonortho_rhs of such a cell.
+template <typename T, int D, int KIND, int NC = CornerData<T, D, KIND>::NC>
+__device__ __forceinline__ void nonortho_rhs_near(const CornerData<T, D, KIND> &cd, int bi, const Near<D> &nr, const int *pin,
+                                                  int f, int flags, bool withVisc, const T *A, T *S) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) S[k] = T(0);
+    const bool direct = flags & NO_DIRECT_RHS, diagonal = flags & NO_DIAGONAL_RHS;
+    if (!(direct || diagonal)) return;
+    const pp_block_desc &b = cd.blocks[bi];
+    const P3 p{pin[0], pin[1], D > 2 ? pin[2] : 0};
+    const T viscP = withVisc ? visc_at<T>(cd.dom, b, f) : T(1);
+    const T raP = (A ? T(1) / A[b.global_offset + f] : T(1)) * viscP;
+    Cross<T, D> cP;
+    cP.load(b, f);
+#pragma unroll
+    for (int face = 0; face < 2 * D; ++face) {
+        const int axis = face >> 1;
+        const int fs = face_sign(face);
+        if (nr.wall[face]) {
+            if (KIND == NK_PRESSURE || cd.neumann(bi, face)) continue;
+            // tangential derivative of the prescribed values along the face
+            const pp_boundary_desc &fb = b.bnd[face];
+            const int ff = face_flat(pin, face, b);
+#pragma unroll
+            for (int dd = 1; dd < D; ++dd) {
+                const int tAxis = (axis + dd) % D;
+                const T bA = fb.has_transform ? lap_coef_t<T, D>(Metric<T, D>::face(fb, ff), tAxis, axis) : T(0);
+                const bool tLo = pin[tAxis] == 0, tHi = pin[tAxis] == b.size[tAxis] - 1;
+                P3 lo = p, hi = p;
+                if (!tLo) lo.add(tAxis, -1);
+                if (!tHi) hi.add(tAxis, 1);
+                const T df = (tLo || tHi) ? T(1.0) : T(0.5);
+                T vh[NC], vl[NC];
+                cd.fixed(bi, face, hi, vh);
+                cd.fixed(bi, face, lo, vl);
+#pragma unroll
+                for (int k = 0; k < NC; ++k) S[k] -= T(fs) * bA * (df * (vh[k] - vl[k])) * viscP;
+            }
+            continue;
+        }
+        const int nf = f + nr.d[face];
+        Cross<T, D> cN;
+        cN.load(b, nf);
+        T raN = A ? T(1) / A[b.global_offset + nf] : T(1);
+        if (withVisc) raN = raN * visc_at<T>(cd.dom, b, nf);
+#pragma unroll
+        for (int dd = 1; dd < D; ++dd) {
+            const int tAxis = (axis + dd) % D;
+            const T faceAlpha = (cP.at(axis, tAxis) * raP + cN.at(axis, tAxis) * raN) * T(0.5);
+            T tg[NC];
+#pragma unroll
+            for (int k = 0; k < NC; ++k) tg[k] = T(0);
+#pragma unroll
+            for (int tUp = 0; tUp < 2; ++tUp) {
+                const int tFace = tAxis * 2 + tUp;
+                const int tfs = face_sign(tFace);
+                if (!nr.wall[tFace]) {
+                    // the corner's value: a quarter of the cells the flags select
+                    T v[NC];
+                    cd.at(bi, f + nr.d[face] + nr.d[tFace], v);
+                    if (direct) {
+                        T vF[NC], vG[NC];
+                        cd.at(bi, f + nr.d[face], vF);
+                        cd.at(bi, f + nr.d[tFace], vG);
+#pragma unroll
+                        for (int k = 0; k < NC; ++k) v[k] = vF[k] + vG[k] + v[k];
+                    }
+#pragma unroll
+                    for (int k = 0; k < NC; ++k) tg[k] += T(tfs) * (v[k] / T(4));
+                } else if (KIND == NK_PRESSURE || cd.neumann(bi, tFace)) {
+                    const int tOther = tFace ^ 1;
+                    if (direct) {
+                        T vF[NC], vO[NC];
+                        cd.at(bi, nf, vF);
+                        cd.at(bi, f + nr.d[tOther], vO);
+#pragma unroll
+                        for (int k = 0; k < NC; ++k) {
+                            tg[k] += T(tfs) * vF[k] * T(0.75);
+                            tg[k] += T(-tfs) * vO[k] * T(0.25);
+                        }
+                    }
+                    if (diagonal) {
+                        T e[NC];
+                        cd.at(bi, nf + nr.d[tOther], e);
+#pragma unroll
+                        for (int k = 0; k < NC; ++k) tg[k] += T(-tfs) * e[k] * T(0.25);
+                    }
+                } else {
+                    // the face's prescribed values, averaged along the step across `face`
+                    T x[NC];
+                    cd.fixed(bi, tFace, p, x);
+                    if (!at_bnd(p, face, b)) {
+                        P3 q = p;
+                        q.add(axis, fs);
+                        T o[NC];
+                        cd.fixed(bi, tFace, q, o);
+#pragma unroll
+                        for (int k = 0; k < NC; ++k) x[k] = (x[k] + o[k]) * T(0.5);
+                    }
+#pragma unroll
+                    for (int k = 0; k < NC; ++k) tg[k] += T(tfs) * x[k];
                 }
             }
 #pragma unroll

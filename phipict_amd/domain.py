@@ -1499,6 +1499,8 @@ class Domain:
         d.scalar_rhs = _lib.ptr(self.scalarRHS) if scalar else None
         d.scalar_result = _lib.ptr(self.scalarResult) if scalar else None
         d.advection_scheme = int(self.advectionScheme)
+        d.unconnected = int(all(min(b.getSizesZYX()) > 1 and not any(isinstance(f, ConnectedBoundary) for f in b.boundaries)
+                                for b in self._blocks))
         self._changed = False
 
     ATLAS_RING = 16
