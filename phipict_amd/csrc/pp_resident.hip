@@ -65,34 +65,6 @@ template <> struct Tagged<float> {
     }
 };
 
-// Sum over the wavefront in every lane, in the order of a shuffle tree over 32, 16, 8, 4, 2, 1 lanes
-// (that of wave_sum): half-wave and row swaps, then DPP row shifts, no LDS round trips.
-__device__ __forceinline__ double join(unsigned hi, unsigned lo) { return __hiloint2double(int(hi), int(lo)); }
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
-    return v + __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double wave_sum0(double v) { // lane 0
-    const unsigned lo = __double2loint(v), hi = __double2hiint(v);
-    const auto l32 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-    const auto h32 = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-    v = join(h32[0], l32[0]) + join(h32[1], l32[1]);
-    const unsigned lo2 = __double2loint(v), hi2 = __double2hiint(v);
-    const auto l16 = __builtin_amdgcn_permlane16_swap(lo2, lo2, false, false);
-    const auto h16 = __builtin_amdgcn_permlane16_swap(hi2, hi2, false, false);
-    v = join(h16[0], l16[0]) + join(h16[1], l16[1]);
-    v = dpp_add<0x108>(v); // row_shl:8
-    v = dpp_add<0x104>(v);
-    v = dpp_add<0x102>(v);
-    return dpp_add<0x101>(v);
-}
-__device__ __forceinline__ double wave_total(double v) {
-    v = wave_sum0(v);
-    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)), __builtin_amdgcn_readfirstlane(__double2loint(v)));
-}
-
 // The value unchanged, opaque to the compiler.
 __device__ __forceinline__ int hide(int v) {
     asm volatile("" : "+v"(v));

@@ -28,15 +28,19 @@
 
 namespace pp {
 
-constexpr int WG = 256; // threads per workgroup of every phase and level kernel
-// Workgroups per CU of the phase kernels (the width every workgroup folds at the start of the
-// next phase) and of the level passes.
-#ifndef PP_PHASE_WG_PER_CU
-#define PP_PHASE_WG_PER_CU 8
-#endif
-#ifndef PP_LEVEL_WG_PER_CU
-#define PP_LEVEL_WG_PER_CU 8
-#endif
+// Threads per workgroup of the phase kernels, the level passes and the segmented solves, and of the
+// passes of AMG-PCG over the finest level. Every workgroup folds the partial set that the previous
+// launch left, one value per workgroup: with 512 of them instead of 2048 the three such launches of
+// an iteration over 663 k rows take 32, 23 and 20 us instead of 35, 28 and 22. The CG and BiCGStab
+// kernels share their rows among several right-hand sides and take the registers of one large
+// workgroup per CU: 1.77 M rows of three right-hand sides take 85 us in the small ones, 91 in the
+// large ones.
+constexpr int WG = 256;
+constexpr int PCG_WG = 1024;
+// Threads per CU of the phase kernels and of the level passes (a half, three eighths and a quarter
+// measured the same or slower: 663 k rows of AMG-PCG 7.39, 7.30 and 7.53 ms for 7.23, BiCGStab on
+// 1.77 M rows 1.34, 1.42 and 2.09 ms for 0.96).
+constexpr int PHASE_THREADS = 2048;
 
 // ======================================================================================
 // Partial sets and the replicated fold
@@ -47,49 +51,70 @@ struct Parts {
     __device__ __forceinline__ double *at(int rhs, int q) const { return p + ((size_t)rhs * nq + q) * G; }
 };
 
-// Write this workgroup's sums acc[k][q] of right-hand sides first..first+count-1.
-template <int NB, int NQ>
+// Write this workgroup's sums acc[k][q] of right-hand sides first..first+count-1 (lds: NT / 64
+// doubles per sum).
+template <int NT, int NB, int NQ>
 __device__ __forceinline__ void put_parts(const Parts &P, double (&acc)[NB][NQ], int first, int count, double *lds) {
-    double flat[NB * NQ];
-#pragma unroll
-    for (int k = 0; k < NB; ++k)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) flat[k * NQ + q] = acc[k][q];
-    block_sum<NB * NQ>(flat, lds);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < count; ++k)
-            for (int q = 0; q < NQ; ++q) P.at(first + k, q)[blockIdx.x] = flat[k * NQ + q];
-}
-
-// Totals of quantities q0..q0+NQ-1 of right-hand sides first..first+count-1, folded over
-// the G partials in a fixed order and broadcast to every thread: every workgroup of a launch
-// obtains the same bits.
-template <int NB, int NQ>
-__device__ __forceinline__ void fold(const Parts &P, int q0, int first, int count, double (&out)[NB][NQ], double *lds) {
-    double acc[NB * NQ];
+    const int t = threadIdx.x;
 #pragma unroll
     for (int k = 0; k < NB; ++k)
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            double s = 0.0;
-            if (k < count) {
-                const double *src = P.at(first + k, q0 + q);
-                for (int g = threadIdx.x; g < P.G; g += WG) s += src[g];
-            }
-            acc[k * NQ + q] = s;
+            const double v = wave_sum0(acc[k][q]);
+            if ((t & 63) == 0) lds[(k * NQ + q) * (NT / 64) + (t >> 6)] = v;
         }
-    block_sum<NB * NQ>(acc, lds);
-    __shared__ double share[16];
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int v = 0; v < NB * NQ; ++v) share[v] = acc[v];
     __syncthreads();
+    if (t < count * NQ) {
+        double v = 0.0;
 #pragma unroll
-    for (int k = 0; k < NB; ++k)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) out[k][q] = share[k * NQ + q];
-    __syncthreads();
+        for (int w = 0; w < NT / 64; ++w) v += lds[t * (NT / 64) + w];
+        P.at(first + t / NQ, t % NQ)[blockIdx.x] = v;
+    }
 }
+
+// Totals of quantities q0..q0+NQ-1 of right-hand sides first..first+count-1, folded over the G
+// partials in a fixed order by one wavefront and left in out[k * NQ + q] (LDS): every workgroup
+// of a launch obtains the same bits. The loads of FOLD_AHEAD strides and of all quantities are in
+// flight together.
+constexpr int FOLD_AHEAD = 8;
+template <int NB, int NQ>
+__device__ __forceinline__ void fold(const Parts &P, int q0, int first, int count, double *out) {
+    const int lane = threadIdx.x & 63;
+    double acc[NB * NQ];
+#pragma unroll
+    for (int v = 0; v < NB * NQ; ++v) acc[v] = 0.0;
+    for (int g0 = lane; g0 < P.G; g0 += FOLD_AHEAD * 64) {
+        double in[NB * NQ][FOLD_AHEAD];
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const double *src = P.at(first + (k < count ? k : 0), q0 + q);
+#pragma unroll
+                for (int u = 0; u < FOLD_AHEAD; ++u) in[k * NQ + q][u] = g0 + 64 * u < P.G ? src[g0 + 64 * u] : 0.0;
+            }
+#pragma unroll
+        for (int v = 0; v < NB * NQ; ++v)
+#pragma unroll
+            for (int u = 0; u < FOLD_AHEAD; ++u) acc[v] += in[v][u];
+    }
+#pragma unroll
+    for (int v = 0; v < NB * NQ; ++v) {
+        const double t = wave_sum0(acc[v]);
+        if (lane == 0) out[v] = t;
+    }
+}
+
+// What a phase kernel's first wavefront decided, for the others: one wavefront folds and applies the
+// rules, several hundred straight instructions that all of them executed before (BiCGStab on 1.77 M
+// rows of three right-hand sides: 958 us with it, 984 without).
+template <int NB, typename T>
+struct Head {
+    double tot[NB * 3], tot2[NB * 3]; // folded sums
+    T step[NB], step2[NB];            // beta, alpha or omega
+    int act[NB], flag[NB];            // still active; the kernel's own mark
+    int any;
+};
 
 // ======================================================================================
 // Row access of the system matrix (shared by NB right-hand sides of one matrix)
@@ -136,26 +161,28 @@ __device__ __forceinline__ void row_each(const Csr<T> &A, const T *__restrict__ 
     }
 }
 
-// Grid-wide row sweep of a phase kernel: workgroup x takes rows x*WG + t, + G*WG, ...
-#define PP_ROWS(i, n) for (int i = blockIdx.x * WG + (int)threadIdx.x; i < (n); i += gridDim.x * WG)
+// Grid-wide row sweep of a phase kernel: workgroup x takes rows x*NT + t, + G*NT, ...
+#define PP_ROWS(i, n) for (int i = blockIdx.x * NT + (int)threadIdx.x; i < (n); i += gridDim.x * NT)
 
-// Records of the span, read into registers.
-template <int NB>
-__device__ __forceinline__ void load_recs(const SolveRec *recs, const Span &sp, SolveRec (&R)[NB], bool (&act)[NB],
-                                          bool &any) {
-    any = false;
-#pragma unroll
+// Runs decide(k, R) for every right-hand side of the span in the first wavefront, on a copy of its
+// record: k's step, flag and whether it stays active go to H, the record to `out` (workgroup 0).
+template <int NB, typename T, typename F>
+__device__ __forceinline__ void decide_each(Head<NB, T> &H, const SolveRec *in, SolveRec *out, const Span &sp, F decide) {
+    const bool lead = threadIdx.x == 0;
+    int any = 0;
+#pragma unroll 1
     for (int k = 0; k < NB; ++k) {
-        if (k < sp.count) R[k] = recs[sp.first + k];
-        act[k] = k < sp.count && rec_active(R[k]);
-        any |= act[k];
+        int act = 0;
+        if (k < sp.count) {
+            SolveRec R = in[sp.first + k];
+            decide(k, R);
+            act = rec_active(R);
+            if (out && blockIdx.x == 0 && lead) out[sp.first + k] = R;
+        }
+        if (lead) H.act[k] = act;
+        any |= act;
     }
-}
-
-template <int NB>
-__device__ __forceinline__ void store_recs(SolveRec *recs, const Span &sp, const SolveRec (&R)[NB]) {
-    if (recs && blockIdx.x == 0 && threadIdx.x == 0)
-        for (int k = 0; k < sp.count; ++k) recs[sp.first + k] = R[k];
+    if (lead) H.any = any;
 }
 
 // Control of a phase kernel, passed by value.
@@ -180,30 +207,31 @@ struct Jac {
 // Opening: partial sums of b, and the initial residual r = b - A x
 // ======================================================================================
 // Partials of sum(v) per right-hand side (the projection of a rank-deficient b).
-template <typename T>
-__global__ void __launch_bounds__(WG) k_sum(const T *__restrict__ v, int n, Parts out) {
-    __shared__ double lds[16];
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_sum(const T *__restrict__ v, int n, Parts out) {
+    __shared__ double lds[NT / 64];
     const int b = blockIdx.y;
     double acc[1][1] = {{0.0}};
     PP_ROWS(i, n) acc[0][0] += double(v[(size_t)b * n + i]);
-    put_parts<1, 1>(out, acc, b, 1, lds);
+    put_parts<NT, 1, 1>(out, acc, b, 1, lds);
 }
 
 // r = bw - A x with bw = b - mean(b) when bSum is given (bw written to bwOut for later
 // residual resets), r0 = r for BiCGStab. Partials: (r, r), (bw, bw) and sum(r), or with the
 // Jacobi preconditioner (r, D^-1 r) in the last place.
-template <typename T, int NB, int EW, bool JAC>
-__global__ void __launch_bounds__(WG) k_open(Csr<T> A, const T *__restrict__ b, Parts bSum, T *__restrict__ bwOut,
+template <typename T, int NB, int EW, bool JAC, int NT>
+__global__ void __launch_bounds__(NT) k_open(Csr<T> A, const T *__restrict__ b, Parts bSum, T *__restrict__ bwOut,
                                              const T *__restrict__ x, T *__restrict__ r, T *__restrict__ r0, int B,
                                              Parts out, Jac<T> jac) {
-    __shared__ double lds[16 * NB * 3];
+    __shared__ double lds[NT / 64 * NB * 3], sums[NB];
     const int n = A.n;
     const Span sp = span_of<NB>(blockIdx.y, A.rpm, B);
     double mean[NB][1];
     if (bSum.p) {
-        fold<NB, 1>(bSum, 0, sp.first, sp.count, mean, lds);
+        if (threadIdx.x < 64) fold<NB, 1>(bSum, 0, sp.first, sp.count, sums);
+        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NB; ++k) mean[k][0] /= double(n);
+        for (int k = 0; k < NB; ++k) mean[k][0] = sums[k] / double(n);
     }
     const T *val = A.val + (size_t)sp.m * A.valStride;
     const T *ellv = A.ell_val + (A.valStride ? (size_t)sp.m * A.ell_w * n : 0);
@@ -234,7 +262,7 @@ __global__ void __launch_bounds__(WG) k_open(Csr<T> A, const T *__restrict__ b, 
                 else acc[k][2] += double(ri);
             }
     }
-    put_parts<NB, 3>(out, acc, sp.first, sp.count, lds);
+    put_parts<NT, NB, 3>(out, acc, sp.first, sp.count, lds);
 }
 
 __global__ void k_init_recs(SolveRec *a, int B, double tol, const double *tols, int maxit) {
@@ -259,38 +287,42 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, T *__restrict__ r, con
                                                 T *__restrict__ pOut, T *__restrict__ q, const T *__restrict__ x,
                                                 const T *__restrict__ bw, Parts rrIn, Parts pqOut, Parts resetOut,
                                                 Phase ph, int mode, Jac<T> jac) {
-    __shared__ double lds[16 * NB * 3];
+    constexpr int NT = WG;
+    __shared__ double lds[NT / 64 * NB * 2];
+    __shared__ Head<NB, T> H;
     const int n = A.n;
     const Span sp = span_of<NB>(blockIdx.y, A.rpm, ph.B);
-    SolveRec R[NB];
-    bool act[NB], any;
-    load_recs<NB>(ph.in, sp, R, act, any);
+    if (threadIdx.x < 64) {
+        if (mode != TURN_AFTER_RESET) fold<NB, 3>(rrIn, 0, sp.first, sp.count, H.tot);
+        decide_each<NB>(H, ph.in, mode == TURN_AFTER_RESET ? nullptr : ph.out, sp, [&](int k, SolveRec &R) {
+            T beta = T(0);
+            if (mode != TURN_AFTER_RESET && rec_active(R)) {
+                const double *tot = H.tot + 3 * k;
+                if (mode == TURN_OPEN) {
+                    rule_open(R, tot[0], ph.scale, false);
+                    R.zero = tot[1] == 0.0;
+                    if (JAC) R.rho = tot[2];
+                } else {
+                    rule_step(R, tot[0], ph.scale, ph.keepBest != 0);
+                    if (rec_active(R)) beta = T(rule_cg_beta(R, JAC ? tot[2] : tot[0]));
+                }
+                if (mode == TURN_STEP_RESET && rec_active(R)) R.flags |= R_FRESH | R_RESET;
+            }
+            if (threadIdx.x == 0) {
+                H.step[k] = beta;
+                H.flag[k] = R.flags & R_FRESH;
+            }
+        });
+    }
+    __syncthreads();
+    const bool any = H.any;
+    bool act[NB], fresh[NB];
     T beta[NB];
 #pragma unroll
-    for (int k = 0; k < NB; ++k) beta[k] = T(0);
-    if (mode != TURN_AFTER_RESET) {
-        double tot[NB][3];
-        fold<NB, 3>(rrIn, 0, sp.first, sp.count, tot, lds);
-        any = false;
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-            if (!act[k]) continue;
-            if (mode == TURN_OPEN) {
-                rule_open(R[k], tot[k][0], ph.scale, false);
-                R[k].zero = tot[k][1] == 0.0;
-                if (JAC) R[k].rho = tot[k][2];
-            } else {
-                rule_step(R[k], tot[k][0], ph.scale, ph.keepBest != 0);
-                if (rec_active(R[k])) beta[k] = T(rule_cg_beta(R[k], JAC ? tot[k][2] : tot[k][0]));
-            }
-            act[k] = rec_active(R[k]);
-            any |= act[k];
-        }
-        if (mode == TURN_STEP_RESET)
-#pragma unroll
-            for (int k = 0; k < NB; ++k)
-                if (act[k]) R[k].flags |= R_FRESH | R_RESET;
-        store_recs<NB>(ph.out, sp, R);
+    for (int k = 0; k < NB; ++k) {
+        act[k] = H.act[k];
+        fresh[k] = act[k] && H.flag[k];
+        beta[k] = act[k] ? H.step[k] : T(0);
     }
     const T *val = A.val + (size_t)sp.m * A.valStride;
     const T *ellv = A.ell_val + (A.valStride ? (size_t)sp.m * A.ell_w * n : 0);
@@ -319,12 +351,9 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, T *__restrict__ r, con
                         if constexpr (JAC) acc[k][1] += double(ri) * double(ri * dv[i]);
                     }
             }
-        put_parts<NB, 2>(resetOut, acc, sp.first, sp.count, lds);
+        put_parts<NT, NB, 2>(resetOut, acc, sp.first, sp.count, lds);
         return;
     }
-    bool fresh[NB];
-#pragma unroll
-    for (int k = 0; k < NB; ++k) fresh[k] = (R[k].flags & R_FRESH) != 0;
     double acc[NB][1];
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k][0] = 0.0;
@@ -353,47 +382,45 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, T *__restrict__ r, con
                     acc[k][0] += double(pi) * double(ap[k]);
                 }
         }
-    put_parts<NB, 1>(pqOut, acc, sp.first, sp.count, lds);
+    put_parts<NT, NB, 1>(pqOut, acc, sp.first, sp.count, lds);
 }
 
 // Advance: alpha = rho / (p', q) from the folded partials; x += alpha p', r -= alpha q
 // (saving x first when it is the best iterate); partials (r, r), 0 and sum(r), or (r, D^-1 r)
 // with JAC. Workgroup 0 commits the records (fresh and reset marks cleared; a reset's rho from
 // resetIn).
-template <typename T, int NB, bool JAC>
-__global__ void __launch_bounds__(WG) k_cg_step(int n, int rpm, T *__restrict__ r, const T *__restrict__ p,
+template <typename T, int NB, bool JAC, int NT>
+__global__ void __launch_bounds__(NT) k_cg_step(int n, int rpm, T *__restrict__ r, const T *__restrict__ p,
                                                 const T *__restrict__ q, T *__restrict__ x, T *__restrict__ xbest,
                                                 Parts pqIn, Parts resetIn, Parts rrOut, Phase ph, Jac<T> jac) {
-    __shared__ double lds[16 * NB * 3];
+    __shared__ double lds[NT / 64 * NB * 3];
+    __shared__ Head<NB, T> H;
     const Span sp = span_of<NB>(blockIdx.y, rpm, ph.B);
-    SolveRec R[NB];
-    bool act[NB], any;
-    load_recs<NB>(ph.in, sp, R, act, any);
-    bool reset = false;
-#pragma unroll
-    for (int k = 0; k < NB; ++k) reset |= act[k] && (R[k].flags & R_RESET);
-    if (reset) {
-        double rr[NB][2];
-        fold<NB, 2>(resetIn, 0, sp.first, sp.count, rr, lds);
-#pragma unroll
-        for (int k = 0; k < NB; ++k)
-            if (act[k] && (R[k].flags & R_RESET)) R[k].rho = JAC ? rr[k][1] : rr[k][0];
+    if (threadIdx.x < 64) {
+        fold<NB, 1>(pqIn, 0, sp.first, sp.count, H.tot);
+        if (resetIn.p) fold<NB, 2>(resetIn, 0, sp.first, sp.count, H.tot2);
+        decide_each<NB>(H, ph.in, ph.out, sp, [&](int k, SolveRec &R) {
+            T alpha = T(0);
+            if (rec_active(R)) {
+                if (R.flags & R_RESET) R.rho = H.tot2[2 * k + (JAC ? 1 : 0)];
+                alpha = T(rule_alpha(R, H.tot[k]));
+                R.flags &= ~(R_FRESH | R_RESET);
+            }
+            if (threadIdx.x == 0) {
+                H.step[k] = alpha;
+                H.flag[k] = xbest && (R.flags & R_KEEP);
+            }
+        });
     }
-    double pq[NB][1];
-    fold<NB, 1>(pqIn, 0, sp.first, sp.count, pq, lds);
+    __syncthreads();
     T alpha[NB];
-    bool keep[NB];
+    bool act[NB], keep[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        alpha[k] = T(0);
-        keep[k] = false;
-        if (!act[k]) continue;
-        alpha[k] = T(rule_alpha(R[k], pq[k][0]));
-        R[k].flags &= ~(R_FRESH | R_RESET);
-        act[k] = rec_active(R[k]);
-        keep[k] = act[k] && xbest && (R[k].flags & R_KEEP);
+        act[k] = H.act[k];
+        alpha[k] = act[k] ? H.step[k] : T(0);
+        keep[k] = act[k] && H.flag[k];
     }
-    store_recs<NB>(ph.out, sp, R);
     double acc[NB][3];
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k][0] = acc[k][1] = acc[k][2] = 0.0;
@@ -413,7 +440,7 @@ __global__ void __launch_bounds__(WG) k_cg_step(int n, int rpm, T *__restrict__ 
             else acc[k][2] += double(ri);
         }
     }
-    put_parts<NB, 3>(rrOut, acc, sp.first, sp.count, lds);
+    put_parts<NT, NB, 3>(rrOut, acc, sp.first, sp.count, lds);
 }
 
 // ======================================================================================
@@ -424,26 +451,32 @@ __global__ void __launch_bounds__(WG) k_cg_step(int n, int rpm, T *__restrict__ 
 template <typename T>
 __global__ void __launch_bounds__(WG) k_bicg_dir(int n, const T *__restrict__ r, T *__restrict__ p, const T *__restrict__ v,
                                                  Parts rrIn, Phase ph, int open) {
-    __shared__ double lds[16 * 2];
+    constexpr int NT = WG;
+    __shared__ Head<1, T> H;
     const int b = blockIdx.y;
-    SolveRec R = ph.in[b];
-    bool act = rec_active(R);
-    double tot[1][2];
-    fold<1, 2>(rrIn, 0, b, 1, tot, lds);
-    T beta = T(0);
-    if (act) {
-        if (open) {
-            rule_open(R, tot[0][0], ph.scale, true);
-            R.zero = tot[0][1] == 0.0;
-        } else {
-            beta = T(rule_bicg_full(R, tot[0][0], tot[0][1], ph.scale));
-        }
-        act = rec_active(R);
+    if (threadIdx.x < 64) {
+        fold<1, 2>(rrIn, 0, b, 1, H.tot);
+        decide_each<1>(H, ph.in, ph.out, Span{0, b, 1}, [&](int, SolveRec &R) {
+            T beta = T(0);
+            if (rec_active(R)) {
+                if (open) {
+                    rule_open(R, H.tot[0], ph.scale, true);
+                    R.zero = H.tot[1] == 0.0;
+                } else {
+                    beta = T(rule_bicg_full(R, H.tot[0], H.tot[1], ph.scale));
+                }
+            }
+            if (threadIdx.x == 0) {
+                H.step[0] = beta;
+                H.step2[0] = T(R.omega);
+                H.flag[0] = R.flags & R_FRESH;
+            }
+        });
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) ph.out[b] = R;
-    if (!act) return;
-    const bool fresh = R.flags & R_FRESH;
-    const T omega = T(R.omega);
+    __syncthreads();
+    if (!H.any) return;
+    const bool fresh = H.flag[0];
+    const T beta = H.step[0], omega = H.step2[0];
     const size_t base = (size_t)b * n;
     if (fresh) PP_ROWS(i, n) p[base + i] = r[base + i];
     else PP_ROWS(i, n) p[base + i] = r[base + i] + beta * (p[base + i] - omega * v[base + i]);
@@ -453,12 +486,16 @@ __global__ void __launch_bounds__(WG) k_bicg_dir(int n, const T *__restrict__ r,
 template <typename T, int NB, int EW, bool JAC>
 __global__ void __launch_bounds__(WG) k_bicg_apply(Csr<T> A, const T *__restrict__ p, T *__restrict__ v,
                                                    const T *__restrict__ r0, Parts r0vOut, Phase ph, Jac<T> jac) {
-    __shared__ double lds[16 * NB];
+    constexpr int NT = WG;
+    __shared__ double lds[NT / 64 * NB];
     const int n = A.n;
     const Span sp = span_of<NB>(blockIdx.y, A.rpm, ph.B);
-    SolveRec R[NB];
-    bool act[NB], any;
-    load_recs<NB>(ph.in, sp, R, act, any);
+    bool act[NB], any = false;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        act[k] = k < sp.count && ph.in[sp.first + (k < sp.count ? k : 0)].fate == F_ACTIVE;
+        any |= act[k];
+    }
     const T *val = A.val + (size_t)sp.m * A.valStride;
     const T *ellv = A.ell_val + (A.valStride ? (size_t)sp.m * A.ell_w * n : 0);
     double acc[NB][1];
@@ -485,7 +522,7 @@ __global__ void __launch_bounds__(WG) k_bicg_apply(Csr<T> A, const T *__restrict
                     acc[k][0] += double(r0[o]) * double(ap[k]);
                 }
         }
-    put_parts<NB, 1>(r0vOut, acc, sp.first, sp.count, lds);
+    put_parts<NT, NB, 1>(r0vOut, acc, sp.first, sp.count, lds);
 }
 
 // alpha = rho / (r0, v) folded; s = r - alpha v (formed at every neighbour as it is read),
@@ -493,23 +530,26 @@ __global__ void __launch_bounds__(WG) k_bicg_apply(Csr<T> A, const T *__restrict
 template <typename T, int NB, int EW, bool JAC>
 __global__ void __launch_bounds__(WG) k_bicg_stab(Csr<T> A, const T *__restrict__ r, const T *__restrict__ v,
                                                   T *__restrict__ t, Parts r0vIn, Parts tsOut, Phase ph, Jac<T> jac) {
-    __shared__ double lds[16 * NB * 3];
+    constexpr int NT = WG;
+    __shared__ double lds[NT / 64 * NB * 3];
+    __shared__ Head<NB, T> H;
     const int n = A.n;
     const Span sp = span_of<NB>(blockIdx.y, A.rpm, ph.B);
-    SolveRec R[NB];
-    bool act[NB], any;
-    load_recs<NB>(ph.in, sp, R, act, any);
-    double r0v[NB][1];
-    fold<NB, 1>(r0vIn, 0, sp.first, sp.count, r0v, lds);
+    if (threadIdx.x < 64) {
+        fold<NB, 1>(r0vIn, 0, sp.first, sp.count, H.tot);
+        decide_each<NB>(H, ph.in, nullptr, sp, [&](int k, SolveRec &R) {
+            const T alpha = rec_active(R) ? T(rule_alpha(R, H.tot[k])) : T(0);
+            if (threadIdx.x == 0) H.step[k] = alpha;
+        });
+    }
+    __syncthreads();
+    const bool any = H.any;
+    bool act[NB];
     T alpha[NB];
-    any = false;
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        alpha[k] = T(0);
-        if (!act[k]) continue;
-        alpha[k] = T(rule_alpha(R[k], r0v[k][0]));
-        act[k] = rec_active(R[k]);
-        any |= act[k];
+        act[k] = H.act[k];
+        alpha[k] = act[k] ? H.step[k] : T(0);
     }
     const T *val = A.val + (size_t)sp.m * A.valStride;
     const T *ellv = A.ell_val + (A.valStride ? (size_t)sp.m * A.ell_w * n : 0);
@@ -541,7 +581,7 @@ __global__ void __launch_bounds__(WG) k_bicg_stab(Csr<T> A, const T *__restrict_
                     acc[k][2] += double(si) * double(si);
                 }
         }
-    put_parts<NB, 3>(tsOut, acc, sp.first, sp.count, lds);
+    put_parts<NT, NB, 3>(tsOut, acc, sp.first, sp.count, lds);
 }
 
 // alpha and omega from the folded partials (half-step test on (s, s)); x += alpha p + omega s,
@@ -552,26 +592,36 @@ __global__ void __launch_bounds__(WG) k_bicg_step(int n, int rpm, T *__restrict_
                                                   const T *__restrict__ p, const T *__restrict__ v,
                                                   const T *__restrict__ t, T *__restrict__ x, Parts r0vIn, Parts tsIn,
                                                   Parts rrOut, Phase ph, Jac<T> jac) {
-    __shared__ double lds[16 * 3];
+    constexpr int NT = WG;
+    __shared__ double lds[NT / 64 * 2];
+    __shared__ Head<1, T> H;
     const int b = blockIdx.y;
-    SolveRec R = ph.in[b];
-    bool act = rec_active(R);
-    double r0v[1][1], ts[1][3];
-    fold<1, 1>(r0vIn, 0, b, 1, r0v, lds);
-    fold<1, 3>(tsIn, 0, b, 1, ts, lds);
-    bool half = false;
-    if (act) {
-        R.alpha = rule_alpha(R, r0v[0][0]);
-        if (rec_active(R)) R.omega = rule_bicg_half(R, ts[0][0], ts[0][1], ts[0][2], ph.scale);
-        act = rec_active(R);
-        half = act && (R.flags & R_HALF);
-        if (half) rule_bicg_half_met(R);
-        R.flags &= ~R_FRESH;
+    if (threadIdx.x < 64) {
+        fold<1, 1>(r0vIn, 0, b, 1, H.tot);
+        fold<1, 3>(tsIn, 0, b, 1, H.tot2);
+        // act: rows to update, also by a half step that ends the solve
+        decide_each<1>(H, ph.in, ph.out, Span{0, b, 1}, [&](int, SolveRec &R) {
+            bool act = rec_active(R), half = false;
+            if (act) {
+                R.alpha = rule_alpha(R, H.tot[0]);
+                if (rec_active(R)) R.omega = rule_bicg_half(R, H.tot2[0], H.tot2[1], H.tot2[2], ph.scale);
+                act = rec_active(R);
+                half = act && (R.flags & R_HALF);
+                if (half) rule_bicg_half_met(R);
+                R.flags &= ~R_FRESH;
+            }
+            if (threadIdx.x == 0) {
+                H.step[0] = T(R.alpha);
+                H.step2[0] = T(R.omega);
+                H.flag[0] = act ? (half ? 2 : 1) : 0;
+            }
+        });
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) ph.out[b] = R;
+    __syncthreads();
     double acc[1][2] = {{0.0, 0.0}};
-    if (act) {
-        const T alpha = T(R.alpha), omega = T(R.omega);
+    if (H.flag[0]) {
+        const bool half = H.flag[0] == 2;
+        const T alpha = H.step[0], omega = H.step2[0];
         const size_t base = (size_t)b * n;
         const T *dv = JAC ? jac.of(b / rpm) : nullptr;
         PP_ROWS(i, n) {
@@ -589,7 +639,7 @@ __global__ void __launch_bounds__(WG) k_bicg_step(int n, int rpm, T *__restrict_
             }
         }
     }
-    put_parts<1, 2>(rrOut, acc, b, 1, lds);
+    put_parts<NT, 1, 2>(rrOut, acc, b, 1, lds);
 }
 
 // Inverse diagonal of each matrix for the Jacobi preconditioner (kInverseDiagonal,
@@ -636,6 +686,7 @@ __global__ void k_take_best(T *x, const T *xbest, const SolveRec *rec, int n, in
 // `lanes` (a power of two <= 32) is chosen per matrix by the autotuner for the sliced layouts
 // and by the row length for plain CSR.
 enum Layout { LAY_CSR = 0, LAY_SELL = 1, LAY_ELL = 2 };
+constexpr int level_threads(int lay) { return lay == LAY_ELL ? PCG_WG : WG; }
 
 template <typename H>
 struct LvMat {
@@ -650,8 +701,14 @@ struct LvMat {
 
 // Sum over row i of M(i, c) * g(c), split over `lanes` lanes of the wavefront (sub-lane j);
 // after the exchange every lane of the row's group holds the total (fixed order).
+// Sliced rows are read SELL_AHEAD entries of a lane at a time (past the slice's end the last one again,
+// not added): the columns and values of a chunk, then its gathers, are each one round trip. Such a
+// pass over a coarse level is a chain of round trips and little else: with the record, the slice and
+// the row's own values out of the chain as well, a restriction or interpolation takes 5.7 us instead
+// of 6.4 (means over the levels of 663 k rows).
+constexpr int SELL_AHEAD = 4;
 template <int LAY, int EW, typename H, typename Gth>
-__device__ __forceinline__ H lv_row(const LvMat<H> &M, const H *__restrict__ val, int i, int j, bool valid, Gth g) {
+__device__ __forceinline__ H lv_row(const LvMat<H> &M, const H *__restrict__ val, int tile, int i, int j, bool valid, Gth g) {
     H sum = H(0);
     if constexpr (LAY == LAY_ELL) {
         if (valid) {
@@ -673,12 +730,22 @@ __device__ __forceinline__ H lv_row(const LvMat<H> &M, const H *__restrict__ val
     } else {
         if (valid) {
             if constexpr (LAY == LAY_SELL) {
-                const int per = 64 / M.lanes;
-                const int s = i / per;
-                const int64_t base = M.off[s] + (int64_t)(i - s * per) * M.lanes + j;
-                const int w = M.steps[s];
-#pragma unroll 4
-                for (int k = 0; k < w; ++k) sum += val[base + 64 * k] * g(M.col[base + 64 * k]);
+                const int64_t base = (int64_t)M.off[tile] + (threadIdx.x & 63); // a slice is a tile
+                const int w = M.steps[tile];
+                for (int k = 0; k < w; k += SELL_AHEAD) {
+                    int c[SELL_AHEAD];
+                    H v[SELL_AHEAD], x[SELL_AHEAD];
+#pragma unroll
+                    for (int u = 0; u < SELL_AHEAD; ++u) {
+                        const int64_t e = base + 64 * min(k + u, w - 1);
+                        c[u] = M.col[e];
+                        v[u] = val[e];
+                    }
+#pragma unroll
+                    for (int u = 0; u < SELL_AHEAD; ++u) x[u] = g(c[u]);
+#pragma unroll
+                    for (int u = 0; u < SELL_AHEAD; ++u) sum = k + u < w ? sum + v[u] * x[u] : sum;
+                }
             } else {
                 const int end = M.row[i + 1];
                 for (int e = M.row[i] + j; e < end; e += M.lanes) sum += val[e] * g(M.col[e]);
@@ -715,59 +782,81 @@ struct LvPass {
     Parts sums;
 };
 
+// The wavefront's index in the launch (uniform: slice offsets and steps are then scalar loads).
+template <int NT>
+__device__ __forceinline__ int first_tile() {
+    return __builtin_amdgcn_readfirstlane((blockIdx.x * NT + (int)threadIdx.x) >> 6);
+}
+
 template <int OP, int LAY, int EW, typename TB, typename H, typename TO>
 __device__ __forceinline__ void level_pass(const LvPass<TB, H, TO> &a, int batch, double shift, double *lds) {
+    constexpr int NT = level_threads(LAY);
     const LvMat<H> &M = a.M;
     const int n = M.n;
     const int lanes = LAY == LAY_ELL ? 1 : M.lanes;
     const int per = 64 / lanes;
     const int lane = threadIdx.x & 63, j = lane % lanes;
-    const int wave = (blockIdx.x * WG + (int)threadIdx.x) >> 6, waves = gridDim.x * (WG / 64);
+    const int wave = first_tile<NT>(), waves = gridDim.x * (NT / 64);
     const H *val = M.val + (size_t)batch * M.valStride;
     const H *d = a.dinv ? a.dinv + (size_t)batch * a.dinvStride : nullptr;
     const TB *b = a.b ? a.b + (size_t)batch * a.bStride : nullptr;
     const H *x = a.x + (size_t)batch * a.xStride;
     TO *out = a.out ? a.out + (size_t)batch * a.outStride : nullptr;
     H *res = a.res ? a.res + (size_t)batch * n : nullptr;
-    auto rhs = [&](int c) { return a.shift ? H(double(b[c]) - shift) : H(b[c]); };
+    auto rhs = [&](TB v) { return a.shift ? H(double(v) - shift) : H(v); };
     double acc[1][2] = {{0.0, 0.0}};
     for (int tile = wave; tile * per < n; tile += waves) {
         const int i = tile * per + lane / lanes;
-        const bool valid = i < n;
+        const bool valid = i < n, own = valid && j == 0;
+        // the row's own values travel with its entries, not after their sum
+        H di = H(0), xi = H(0);
+        TB bi = TB(0);
+        TO oi = TO(0);
+        if (own) {
+            if constexpr (OP == OP_FIRST || OP == OP_SWEEP) di = d[i];
+            if constexpr (OP != OP_APPLY) bi = b[i];
+            if constexpr (OP == OP_SWEEP) xi = x[i];
+            if constexpr (OP == OP_APPLY)
+                if (a.accumulate) oi = out[i];
+        }
+        const H s = lv_row<LAY, EW>(M, val, tile, i, j, valid, [&](int c) {
+            if constexpr (OP == OP_FIRST) return d[c] * rhs(b[c]);
+            else return x[c];
+        });
+        if (!own) continue;
         if constexpr (OP == OP_FIRST) {
-            const H s = lv_row<LAY, EW>(M, val, i, j, valid, [&](int c) { return d[c] * rhs(c); });
-            if (valid && j == 0) {
-                const H bi = rhs(i);
-                out[i] = TO(a.omega * d[i] * bi);
-                res[i] = bi - a.omega * s;
-            }
+            const H f = rhs(bi);
+            out[i] = TO(a.omega * di * f);
+            res[i] = f - a.omega * s;
         } else if constexpr (OP == OP_SWEEP) {
-            const H s = lv_row<LAY, EW>(M, val, i, j, valid, [&](int c) { return x[c]; });
-            if (valid && j == 0) {
-                const TO o = TO(x[i] + a.omega * d[i] * (rhs(i) - s));
-                out[i] = o;
-                if (a.sums.p) {
-                    acc[0][0] += double(b[i]) * double(o);
-                    acc[0][1] += double(o);
-                }
+            const TO o = TO(xi + a.omega * di * (rhs(bi) - s));
+            out[i] = o;
+            if (a.sums.p) {
+                acc[0][0] += double(bi) * double(o);
+                acc[0][1] += double(o);
             }
         } else if constexpr (OP == OP_RESID) {
-            const H s = lv_row<LAY, EW>(M, val, i, j, valid, [&](int c) { return x[c]; });
-            if (valid && j == 0) res[i] = rhs(i) - s;
+            res[i] = rhs(bi) - s;
         } else {
-            const H s = lv_row<LAY, EW>(M, val, i, j, valid, [&](int c) { return x[c]; });
-            if (valid && j == 0) out[i] = a.accumulate ? TO(out[i] + s) : TO(s);
+            out[i] = a.accumulate ? TO(oi + s) : TO(s);
         }
     }
     if constexpr (OP == OP_SWEEP)
-        if (a.sums.p) put_parts<1, 2>(a.sums, acc, batch, 1, lds);
+        if (a.sums.p) put_parts<NT, 1, 2>(a.sums, acc, batch, 1, lds);
 }
 
 template <int OP, int LAY, int EW, typename TB, typename H, typename TO>
-__global__ void __launch_bounds__(WG) k_level(LvPass<TB, H, TO> a) {
-    __shared__ double lds[32];
+__global__ void __launch_bounds__(level_threads(LAY)) k_level(LvPass<TB, H, TO> a) {
+    __shared__ double lds[level_threads(LAY) / 64 * 2];
     const int batch = blockIdx.y;
-    if (!rec_active(a.rec[batch])) return;
+    bool live = rec_active(a.rec[batch]);
+    if constexpr (LAY == LAY_SELL) {
+        // The first slice's length is read with the record, not after it: the test of both (a length is
+        // never negative) keeps the two loads together.
+        const int per = 64 / a.M.lanes;
+        live = live & (a.M.steps[min(first_tile<WG>(), (a.M.n - 1) / per)] >= 0);
+    }
+    if (!live) return;
     level_pass<OP, LAY, EW>(a, batch, a.shift ? a.shift[batch] : 0.0, lds);
 }
 
@@ -780,33 +869,34 @@ __global__ void __launch_bounds__(WG) k_level(LvPass<TB, H, TO> a) {
 // residual's mean for the projection (meanOut), then the finest level's first Jacobi sweep
 // with residual.
 template <int LAY, int EW, typename T, typename H>
-__global__ void __launch_bounds__(WG) k_pcg_decide(LvPass<T, H, H> a, Parts rrIn, Parts pqIn, Phase ph, double *meanOut,
+__global__ void __launch_bounds__(level_threads(LAY)) k_pcg_decide(LvPass<T, H, H> a, Parts rrIn, Parts pqIn, Phase ph, double *meanOut,
                                                    int project, int open) {
-    __shared__ double lds[32];
+    __shared__ Head<1, double> hd;
     const int b = blockIdx.y;
-    SolveRec R = ph.in[b];
-    bool act = rec_active(R);
-    double rr[1][3];
-    fold<1, 3>(rrIn, 0, b, 1, rr, lds);
-    if (act) {
-        if (open) rule_open(R, rr[0][0], ph.scale, false);
-        else {
-            double pq[1][1];
-            fold<1, 1>(pqIn, 0, b, 1, pq, lds);
-            SolveRec probe = R;
-            (void)rule_alpha(probe, pq[0][0]);
-            if (!rec_active(probe)) R = probe;
-            else rule_step(R, rr[0][0], ph.scale, ph.keepBest != 0);
-        }
-        act = rec_active(R);
+    if (threadIdx.x < 64) {
+        fold<1, 3>(rrIn, 0, b, 1, hd.tot);
+        if (!open) fold<1, 1>(pqIn, 0, b, 1, hd.tot2);
+        decide_each<1>(hd, ph.in, ph.out, Span{0, b, 1}, [&](int, SolveRec &R) {
+            if (rec_active(R)) {
+                if (open) rule_open(R, hd.tot[0], ph.scale, false);
+                else {
+                    // the step length of the update: a non-finite one ends the solve there
+                    const double alpha = R.rho / hd.tot2[0];
+                    if (!isfinite(alpha)) (void)rule_alpha(R, hd.tot2[0]);
+                    else rule_step(R, hd.tot[0], ph.scale, ph.keepBest != 0);
+                }
+            }
+            const double mean = project ? hd.tot[2] / double(a.M.n) : 0.0;
+            if (threadIdx.x == 0) {
+                hd.step[0] = mean;
+                if (blockIdx.x == 0) meanOut[b] = mean;
+            }
+        });
     }
-    const double mean = project ? rr[0][2] / double(a.M.n) : 0.0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ph.out[b] = R;
-        meanOut[b] = mean;
-    }
-    if (!act) return;
-    level_pass<OP_FIRST, LAY, EW>(a, b, mean, lds);
+    __syncthreads();
+    if (!hd.any) return;
+    const double mean = hd.step[0];
+    level_pass<OP_FIRST, LAY, EW>(a, b, mean, nullptr);
 }
 
 // Direction of the preconditioned solve: rho = (r, z) with z = u - mean(u) (projection) or
@@ -814,35 +904,43 @@ __global__ void __launch_bounds__(WG) k_pcg_decide(LvPass<T, H, H> a, Parts rrIn
 // update (sum(r)); then p' = z + beta pIn (z when fresh) formed at every neighbour as it is
 // read, q = A p', partials (p', q). Workgroup 0 writes the records with rho (fresh cleared).
 template <typename T, int EW>
-__global__ void __launch_bounds__(WG) k_pcg_dir(Csr<T> A, const T *__restrict__ u, const T *__restrict__ pIn,
+__global__ void __launch_bounds__(PCG_WG) k_pcg_dir(Csr<T> A, const T *__restrict__ u, const T *__restrict__ pIn,
                                                 T *__restrict__ pOut, T *__restrict__ q, Parts postIn, Parts rrIn,
                                                 Parts pqOut, Phase ph, int project) {
-    __shared__ double lds[32];
+    constexpr int NT = PCG_WG;
+    __shared__ double lds[NT / 64];
+    __shared__ Head<1, T> H;
     const int n = A.n;
     const int b = blockIdx.y;
-    SolveRec R = ph.in[b];
-    bool act = rec_active(R);
-    double ru[1][2];
-    fold<1, 2>(postIn, 0, b, 1, ru, lds);
-    double zmean = 0.0, rz = ru[0][0];
-    if (project) {
-        double rs[1][1];
-        fold<1, 1>(rrIn, 2, b, 1, rs, lds);
-        zmean = ru[0][1] / double(n);
-        rz = ru[0][0] - zmean * rs[0][0];
+    if (threadIdx.x < 64) {
+        fold<1, 2>(postIn, 0, b, 1, H.tot);
+        if (project) fold<1, 1>(rrIn, 2, b, 1, H.tot2);
+        decide_each<1>(H, ph.in, ph.out, Span{0, b, 1}, [&](int, SolveRec &R) {
+            double zmean = 0.0, rz = H.tot[0];
+            if (project) {
+                zmean = H.tot[1] / double(n);
+                rz = H.tot[0] - zmean * H.tot2[0];
+            }
+            T beta = T(0);
+            int fresh = 0;
+            if (rec_active(R)) {
+                fresh = R.flags & R_FRESH;
+                beta = T(rule_pcg_rho(R, rz));
+                R.flags &= ~R_FRESH;
+            }
+            if (threadIdx.x == 0) {
+                H.step[0] = beta;
+                H.step2[0] = T(zmean);
+                H.flag[0] = fresh;
+            }
+        });
     }
-    T beta = T(0);
-    bool fresh = false;
-    if (act) {
-        fresh = R.flags & R_FRESH;
-        beta = T(rule_pcg_rho(R, rz));
-        R.flags &= ~R_FRESH;
-        act = rec_active(R);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) ph.out[b] = R;
+    __syncthreads();
+    const bool act = H.any, fresh = H.flag[0];
+    const T beta = H.step[0], zmean = H.step2[0];
     double acc[1][1] = {{0.0}};
     if (act) {
-        const T zs = T(zmean);
+        const T zs = zmean;
         const T *val = A.val + (size_t)b * A.valStride;
         const T *ellv = A.ell_val + (A.valStride ? (size_t)b * A.ell_w * n : 0);
         const size_t base = (size_t)b * n;
@@ -859,7 +957,7 @@ __global__ void __launch_bounds__(WG) k_pcg_dir(Csr<T> A, const T *__restrict__ 
             acc[0][0] += double(pi) * double(ap);
         }
     }
-    put_parts<1, 1>(pqOut, acc, b, 1, lds);
+    put_parts<NT, 1, 1>(pqOut, acc, b, 1, lds);
 }
 
 // Dense coarse solve x = pinv b: one wavefront per row of the pseudo-inverse.
@@ -1111,12 +1209,12 @@ static int cu_count() {
     return cus;
 }
 
-// Workgroups per grid row of a phase kernel: enough for every row, at most 8 per CU shared by
+// Workgroups per grid row of a phase kernel: enough for every row, at most PHASE_THREADS per CU shared by
 // the grid rows (the partial sets are folded by every workgroup of the next launch, so the
 // width also bounds the fold).
-static int phase_width(long rows, int gridRows) {
-    const long want = std::max<long>(1, (rows + WG - 1) / WG);
-    const long cap = std::max<long>(1, (long)cu_count() * PP_PHASE_WG_PER_CU / std::max(1, gridRows));
+static int phase_width(long rows, int gridRows, int nt) {
+    const long want = std::max<long>(1, (rows + nt - 1) / nt);
+    const long cap = std::max<long>(1, (long)cu_count() * (PHASE_THREADS / nt) / std::max(1, gridRows));
     return (int)std::min(want, cap);
 }
 
@@ -1430,7 +1528,7 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
     const int NBv = std::min(A.rpm, 4);
     const int numMat = (B + A.rpm - 1) / A.rpm;
     const int rows = numMat * ((A.rpm + NBv - 1) / NBv);
-    const int G = phase_width(n, rows);
+    const int G = phase_width(n, rows, WG);
     enum { V_R = 0, V_Q, V_P0, V_P1, V_XB, V_BW, V_COUNT };
     const size_t vecBytes = sizeof(T) * ((size_t)V_COUNT * n * B + (size_t)numMat * n);
     const size_t partDoubles = (size_t)B * G * (1 + 3 + 1 + 2);
@@ -1447,10 +1545,10 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
     const dim3 grid(G, rows), block(WG);
     hipLaunchKernelGGL(k_init_recs, dim3(1), dim3(64), 0, s, ra, B, tols[0], ntols > 1 ? (const double *)sp.tols : nullptr, maxit);
     if (jacobi) launch_jacobi<T>(A, numMat, V(V_COUNT), s);
-    if (project) hipLaunchKernelGGL((k_sum<T>), dim3(G, B), block, 0, s, b, n, sSum);
+    if (project) hipLaunchKernelGGL((k_sum<T, WG>), dim3(G, B), block, 0, s, b, n, sSum);
     const Phase openPh{ra, rb, B, scale, returnBest};
     PP_JAC_CASE(jacobi, PP_NB_CASE(NBv, PP_EW_CASE(A.ell_w,
-        hipLaunchKernelGGL((k_open<T, NB, EW, JAC>), grid, block, 0, s, A, b, project ? sSum : Parts{nullptr, 1, G},
+        hipLaunchKernelGGL((k_open<T, NB, EW, JAC, WG>), grid, block, 0, s, A, b, project ? sSum : Parts{nullptr, 1, G},
                            project ? bw : (T *)nullptr, x, r, (T *)nullptr, B, sRR, jac);
         hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, 0, s, A, r, p[0], p[1], q, x, bw, sRR, sPQ, sRst,
                            openPh, (int)TURN_OPEN, jac))));
@@ -1462,7 +1560,7 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
         const bool reset = resetEvery > 0 && (j + 1) % resetEvery == 0;
         PP_JAC_CASE(jacobi, PP_NB_CASE(NBv,
             PP_TIMED(PP_K_CG_UPDATE, n, st,
-                hipLaunchKernelGGL((k_cg_step<T, NB, JAC>), grid, block, 0, st, n, A.rpm, r, p[cur], q, x, xbest, sPQ,
+                hipLaunchKernelGGL((k_cg_step<T, NB, JAC, WG>), grid, block, 0, st, n, A.rpm, r, p[cur], q, x, xbest, sPQ,
                                    sRst, sRR, stepPh, jac));
             PP_EW_CASE(A.ell_w,
                 if (reset) {
@@ -1500,7 +1598,7 @@ static int bicg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const
     const int NBv = std::min(A.rpm, 4);
     const int numMat = (B + A.rpm - 1) / A.rpm;
     const int rows = numMat * ((A.rpm + NBv - 1) / NBv);
-    const int G = phase_width(n, std::max(rows, B));
+    const int G = phase_width(n, std::max(rows, B), WG);
     enum { V_R = 0, V_R0, V_P, V_V, V_T, V_COUNT };
     const size_t vecBytes = sizeof(T) * ((size_t)V_COUNT * n * B + (size_t)numMat * n);
     const size_t partDoubles = (size_t)B * G * (3 + 1 + 3);
@@ -1516,7 +1614,7 @@ static int bicg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const
     hipLaunchKernelGGL(k_init_recs, dim3(1), dim3(64), 0, s, ra, B, tols[0], ntols > 1 ? (const double *)sp.tols : nullptr, maxit);
     if (jacobi) launch_jacobi<T>(A, numMat, V(V_COUNT), s);
     PP_NB_CASE(NBv, PP_EW_CASE(A.ell_w,
-        hipLaunchKernelGGL((k_open<T, NB, EW, false>), grid, block, 0, s, A, b, Parts{nullptr, 1, G}, (T *)nullptr, x, r, r0, B,
+        hipLaunchKernelGGL((k_open<T, NB, EW, false, WG>), grid, block, 0, s, A, b, Parts{nullptr, 1, G}, (T *)nullptr, x, r, r0, B,
                            sRR, jac)));
     hipLaunchKernelGGL((k_bicg_dir<T>), gridB, block, 0, s, n, r, p, v, sRR, Phase{ra, rb, B, scale, 0}, 1);
     PP_LAUNCH_CHECK();
@@ -1756,8 +1854,9 @@ template <typename H>
 static dim3 level_grid(const LvMat<H> &M, int lay, int B) {
     const int per = lay == LAY_ELL ? 64 : 64 / M.lanes;
     const long waves = (M.n + per - 1) / per;
-    const long wgs = std::max<long>(1, (waves + WG / 64 - 1) / (WG / 64));
-    return dim3((unsigned)std::min<long>(wgs, std::max(1, cu_count() * PP_LEVEL_WG_PER_CU / B)), B);
+    const int nt = level_threads(lay);
+    const long wgs = std::max<long>(1, (waves + nt / 64 - 1) / (nt / 64));
+    return dim3((unsigned)std::min<long>(wgs, std::max(1, cu_count() * (PHASE_THREADS / nt) / B)), B);
 }
 
 template <int OP, typename TB, typename H, typename TO>
@@ -1765,9 +1864,9 @@ static void launch_level(const LvPass<TB, H, TO> &a, int lay, int B, hipStream_t
     const dim3 g = level_grid(a.M, lay, B);
     if (lay == LAY_SELL) hipLaunchKernelGGL((k_level<OP, LAY_SELL, 0, TB, H, TO>), g, dim3(WG), 0, s, a);
     else if (lay == LAY_CSR) hipLaunchKernelGGL((k_level<OP, LAY_CSR, 0, TB, H, TO>), g, dim3(WG), 0, s, a);
-    else if (a.M.ellW == 7) hipLaunchKernelGGL((k_level<OP, LAY_ELL, 7, TB, H, TO>), g, dim3(WG), 0, s, a);
-    else if (a.M.ellW == 5) hipLaunchKernelGGL((k_level<OP, LAY_ELL, 5, TB, H, TO>), g, dim3(WG), 0, s, a);
-    else hipLaunchKernelGGL((k_level<OP, LAY_ELL, 0, TB, H, TO>), g, dim3(WG), 0, s, a);
+    else if (a.M.ellW == 7) hipLaunchKernelGGL((k_level<OP, LAY_ELL, 7, TB, H, TO>), g, dim3(PCG_WG), 0, s, a);
+    else if (a.M.ellW == 5) hipLaunchKernelGGL((k_level<OP, LAY_ELL, 5, TB, H, TO>), g, dim3(PCG_WG), 0, s, a);
+    else hipLaunchKernelGGL((k_level<OP, LAY_ELL, 0, TB, H, TO>), g, dim3(PCG_WG), 0, s, a);
 }
 
 template <typename T, typename H>
@@ -1777,10 +1876,10 @@ static void launch_decide(const LvPass<T, H, H> &a, int lay, const Parts &rr, co
     if (lay == LAY_CSR)
         hipLaunchKernelGGL((k_pcg_decide<LAY_CSR, 0, T, H>), g, dim3(WG), 0, s, a, rr, pq, ph, means, project, open);
     else if (a.M.ellW == 7)
-        hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 7, T, H>), g, dim3(WG), 0, s, a, rr, pq, ph, means, project, open);
+        hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 7, T, H>), g, dim3(PCG_WG), 0, s, a, rr, pq, ph, means, project, open);
     else if (a.M.ellW == 5)
-        hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 5, T, H>), g, dim3(WG), 0, s, a, rr, pq, ph, means, project, open);
-    else hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 0, T, H>), g, dim3(WG), 0, s, a, rr, pq, ph, means, project, open);
+        hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 5, T, H>), g, dim3(PCG_WG), 0, s, a, rr, pq, ph, means, project, open);
+    else hipLaunchKernelGGL((k_pcg_decide<LAY_ELL, 0, T, H>), g, dim3(PCG_WG), 0, s, a, rr, pq, ph, means, project, open);
 }
 
 template <typename T, typename H>
@@ -1815,7 +1914,7 @@ static int amg_pcg(const Csr<T> &Af, const pp_amg_level *lv, int L, const H *pin
         if (v.p_sell.slice_off) { MP[l] = lv_sell<H>(v.p_sell, v.n, false); layP[l] = LAY_SELL; }
         else { MP[l] = lv_csr<H>(v.p_row, v.p_col, v.p_val, v.n, v.nnz_p, 0); layP[l] = LAY_CSR; }
     }
-    const int G = phase_width(n, B);
+    const int G = phase_width(n, B, PCG_WG);
     const int G0 = (int)level_grid(MA[0], layA[0], B).x;
     enum { V_R = 0, V_Q, V_P0, V_P1, V_U, V_XB, V_COUNT };
     const size_t partDoubles = (size_t)B * G * (1 + 3 + 1) + (size_t)B * 2 * G0;
@@ -1997,9 +2096,9 @@ static int amg_pcg(const Csr<T> &Af, const pp_amg_level *lv, int L, const H *pin
         }
     };
     hipLaunchKernelGGL(k_init_recs, dim3(1), dim3(64), 0, s, ra, B, tols[0], ntols > 1 ? (const double *)sp.tols : nullptr, maxit);
-    if (project) hipLaunchKernelGGL((k_sum<T>), dim3(G, B), dim3(WG), 0, s, b, n, sSum);
+    if (project) hipLaunchKernelGGL((k_sum<T, PCG_WG>), dim3(G, B), dim3(PCG_WG), 0, s, b, n, sSum);
     PP_EW_CASE(Af.ell_w,
-        hipLaunchKernelGGL((k_open<T, 1, EW, false>), dim3(G, B), dim3(WG), 0, s, Af, b, project ? sSum : Parts{nullptr, 1, G},
+        hipLaunchKernelGGL((k_open<T, 1, EW, false, PCG_WG>), dim3(G, B), dim3(PCG_WG), 0, s, Af, b, project ? sSum : Parts{nullptr, 1, G},
                            (T *)nullptr, x, r, (T *)nullptr, B, sRR, Jac<T>{nullptr, 0}));
     decide(s, Phase{ra, rb, B, scale, returnBest}, 1);
     PP_LAUNCH_CHECK();
@@ -2010,10 +2109,10 @@ static int amg_pcg(const Csr<T> &Af, const pp_amg_level *lv, int L, const H *pin
         vcycle_rest(st);
         PP_TIMED(PP_K_PCG_DIRECTION, n, st,
             PP_EW_CASE(Af.ell_w,
-                hipLaunchKernelGGL((k_pcg_dir<T, EW>), dim3(G, B), dim3(WG), 0, st, Af, u, p[cur2], p[cur2 ^ 1], q, sPost, sRR,
+                hipLaunchKernelGGL((k_pcg_dir<T, EW>), dim3(G, B), dim3(PCG_WG), 0, st, Af, u, p[cur2], p[cur2 ^ 1], q, sPost, sRR,
                                    sPQ, dirPh, project)));
         PP_TIMED(PP_K_PCG_UPDATE, n, st,
-            hipLaunchKernelGGL((k_cg_step<T, 1, false>), dim3(G, B), dim3(WG), 0, st, n, 1, r, p[cur2 ^ 1], q, x, xbest,
+            hipLaunchKernelGGL((k_cg_step<T, 1, false, PCG_WG>), dim3(G, B), dim3(PCG_WG), 0, st, n, 1, r, p[cur2 ^ 1], q, x, xbest,
                                sPQ, Parts{nullptr, 2, G}, sRR, updPh, Jac<T>{nullptr, 0}));
         decide(st, decPh, 0);
     };
