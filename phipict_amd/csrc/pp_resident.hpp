@@ -50,7 +50,5 @@ inline int resident_local_rows(int ew) { return (ew == 5 ? 4 : 3) * RES_LOCAL_WG
 // to R rows per thread; otherwise teams of RES_WG-thread workgroups with R rows per thread.
 template <typename T>
 int launch_resident_cg(const ResArgs<T> &a, int ew, int R, int threads, bool local, hipStream_t s);
-template <typename T>
-int launch_resident_bicg(const ResArgs<T> &a, int ew, int R, int threads, bool local, hipStream_t s);
 
 } // namespace pp
