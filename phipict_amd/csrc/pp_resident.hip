@@ -13,8 +13,12 @@
 // the tag of this exchange, so no ordering between different words is needed and no cache is
 // written back or invalidated (an agent-scope fence in every wave of 256 workgroups measured 30 us).
 // Tags grow from exchange to exchange and from solve to solve, so stale words never match.
-// A word is rewritten two exchanges later at the earliest (two parities), and every team member has
-// then passed an all-gather it could only pass after the readers of the old word were done with it.
+// Every tag has exactly one all-gather, of the sums of that exchange (of nothing where only a vector
+// is exchanged, at a residual replacement). A word is rewritten two tags later at the earliest (two
+// parities). Its writer has then passed the all-gather of the tag between, to which every member
+// contributes only when it is done with the words of the tag before: it has passed that tag's
+// all-gather and read the vector published with it. Without the all-gather at a replacement a member that
+// waits for its stencil neighbours' x alone would overwrite sums that a member farther away still polls.
 //
 // A team member that waits too long (RES_SPINS polls: some other process or a fault keeps a
 // workgroup of the team from running) gives up, and says so in the launch's `failed` word: the host then
@@ -395,9 +399,11 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
         bool fresh = L.out.fresh;
         if (L.out.half) {
             // residual replacement: r = b - A x, a fresh direction
+            // (an all-gather of nothing under the tag of the published x, see the top of the file)
             publish(x);
-            const unsigned xtag = ++tm.tag;
-            __syncthreads();
+            const double none[1] = {0.0};
+            if (!team_decide<1, LOCAL>(tm, none, L, [](const double (&)[1], SolveRec &, Verdict &) {})) return give_up(a);
+            const unsigned xtag = tm.tag;
             double s[2] = {0.0, 0.0};
             T z[R];
 #pragma unroll

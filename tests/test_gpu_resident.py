@@ -85,6 +85,14 @@ def test_resident_cg_options(shape, opts):
     _check(*_grid_operator(shape), 2, np.float64, **opts)
 
 
+@pytest.mark.parametrize("shape", [(512, 256), (331, 396), (71, 60, 62)], ids=["256x1", "129x2", "129x4"])
+def test_residual_replacement_in_large_teams(shape):
+    """Teams whose members poll the sums in two rounds (more than 128 workgroups), with one, two and four rows
+    per thread: replacements exchange x between members that are not neighbours of each other's rows."""
+    print(f"[resident] replacement {shape}", flush=True)
+    _check(*_grid_operator(shape), 1, np.float64, residualResetSteps=7)
+
+
 @pytest.mark.parametrize("n", [2000, 9000])
 def test_rows_beyond_the_kernels_take_another_engine(n):
     """One row of 13 entries among rows of five: no rows dropped."""
