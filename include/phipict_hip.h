@@ -414,6 +414,12 @@ int pp_solve_linear_noalloc(const pp_csr *A, const void *rhs, void *x, int32_t n
                             int32_t use_bicg, int32_t matrix_rank_deficient, int32_t residual_reset_steps,
                             int32_t transpose_a, int32_t return_best, void *stream, pp_solve_result *results);
 
+/* Diagnostic (no reference counterpart): how often a CG solve of the calling host thread went to the
+ * resident engine so far, counts[3] = solves it finished, solves it declined (a matrix row longer than
+ * its kernels take) and solves it gave up on (a workgroup waited too long for another). Declined and
+ * given-up solves were then run by the multi-launch engines. */
+int pp_resident_counts(int64_t *counts);
+
 /* replaces ReleaseKrylovWorkspaces (bindings.cpp:777, krylov.cu:921-924). */
 int pp_release_workspaces(void);
 

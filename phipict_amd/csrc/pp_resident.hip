@@ -263,6 +263,10 @@ template <typename T>
 __device__ __forceinline__ void give_up(const ResArgs<T> &a) {
     if (threadIdx.x == 0) *a.failed = a.done;
 }
+template <typename T>
+__device__ __forceinline__ void decline(const ResArgs<T> &a) {
+    if (threadIdx.x == 0) *a.declined = a.done;
+}
 
 // CG (with dinv its Jacobi variant), a team per right-hand side.
 template <typename T, int EW, int R, bool LOCAL>
@@ -301,7 +305,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
                 o.step = tot[1] / double(sh.n);
             }))
             return give_up(a);
-        if (!L.out.active) return give_up(a);
+        if (!L.out.active) return decline(a);
         if (a.project) mean = T(L.out.step);
     }
     auto rhs = [&](int k) { return a.project ? a.b[v0 + k * blk] - mean : a.b[v0 + k * blk]; };

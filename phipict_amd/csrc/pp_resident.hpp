@@ -30,7 +30,8 @@ struct ResArgs {
     size_t vecLen, zorigin;      // values per parity; vector offset of the first of them
     SolveRec *recs;              // final records
     unsigned *status;            // per right-hand side: `done` from the team that finished it
-    unsigned *failed;            // `done` from a workgroup that gave up
+    unsigned *failed;            // `done` from a workgroup that gave up waiting
+    unsigned *declined;          // `done` from a workgroup whose team has a row longer than the kernel takes
     unsigned tag, done;          // the exchanges' first tag less one; the launch's word
     int n, rpm, G, team0;        // plain solve: rows, right-hand sides per matrix, workgroups per team, first team
     int wgs;                     // workgroups of the launch

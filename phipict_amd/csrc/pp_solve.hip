@@ -1175,6 +1175,7 @@ struct ThreadSpaces {
     SegSpace seg;
     void *tbuf = nullptr; size_t tcap = 0;
     int *tbad = nullptr;
+    int64_t resident[3] = {0, 0, 0}; // solves the resident engine finished, declined and gave up on
 };
 static std::vector<ThreadSpaces *> g_all_spaces; // every thread's, for pp_release_workspaces
 
@@ -1721,24 +1722,29 @@ constexpr int RES_MAXIT = 1 << 26; // above it the tags of one solve could wrap
 static uint32_t resident_tags(int maxit) { return (uint32_t)(4 * ((int64_t)maxit + 4)); }
 
 // Where a resident solve of B right-hand sides leaves its records, then (in the second record copy's
-// place) a word per team and one for failures, told from older contents by this solve's value.
+// place) a word per team, one for teams that gave up and one for teams that declined, told from older
+// contents by this solve's value.
 template <typename T>
 static void resident_status(Space &sp, int B, ResArgs<T> *a) {
     a->recs = recs_a(sp);
     a->status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
     a->failed = a->status + B;
+    a->declined = a->status + B + 1;
     a->done = 0xC0DE0000u + (++sp.solves & 0xffffu);
 }
 
-// All of it back in one copy; *ran: every team finished.
+// All of it back in one copy; *ran: every team finished (counted, with the ways it can fail, for the
+// calling thread).
 template <typename T>
 static int resident_results(Space &sp, int B, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran) {
-    PP_HIP(hipMemcpyAsync(sp.snap, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 1), hipMemcpyDeviceToHost, s));
+    PP_HIP(hipMemcpyAsync(sp.snap, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 2), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     *recs = reinterpret_cast<const SolveRec *>(sp.snap);
     const unsigned *st = reinterpret_cast<const unsigned *>(sp.snap + sizeof(SolveRec) * B);
-    *ran = st[B] != a.done;
+    const bool declined = st[B + 1] == a.done;
+    *ran = st[B] != a.done && !declined;
     for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
+    ++my_spaces().resident[*ran ? 0 : (declined ? 1 : 2)];
     return PP_OK;
 }
 
@@ -2991,6 +2997,12 @@ int pp_amg_pcg_solve(const pp_csr *A, const pp_amg_level *levels, int32_t num_le
 #undef PP_AMG_CALL
     set_error("pp_amg_pcg_solve: unsupported (dtype, hierarchy dtype) combination");
     return PP_ERR_UNSUPPORTED;
+}
+
+int pp_resident_counts(int64_t *counts) {
+    PP_CHECK_ARG(counts, "null argument");
+    for (int k = 0; k < 3; ++k) counts[k] = my_spaces().resident[k];
+    return PP_OK;
 }
 
 int pp_release_workspaces(void) {

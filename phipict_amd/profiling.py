@@ -45,6 +45,15 @@ def start(sample_every: int = 1) -> None:
     _lib.call("pp_kernel_timer_start", int(sample_every))
 
 
+def resident_counts() -> tuple:
+    """CG solves of the calling host thread on the resident engine so far: finished, declined (a row
+    longer than its kernels take) and given up (a workgroup waited too long); the latter two were then
+    run by the multi-launch engines."""
+    counts = np.zeros(3, np.int64)
+    _lib.call("pp_resident_counts", counts.ctypes.data)
+    return tuple(int(c) for c in counts)
+
+
 def stop() -> None:
     _lib.call("pp_kernel_timer_stop")
 

@@ -5,8 +5,13 @@ kernels take (handed to the other engines).
 
 Tolerances: the engine sums in another order than the oracle, so a solve may stop an iteration
 earlier or later; the solutions then differ by what the stopping residual leaves open, which for these
-shifted operators (smallest eigenvalue >= shift) is at most sqrt(n) tol / shift in the 2-norm."""
+shifted operators (smallest eigenvalue >= shift) is at most sqrt(n) tol / shift in the 2-norm.
+
+Every test states which engine the solve came from, by the library's counts of resident solves finished,
+declined and given up."""
 from __future__ import annotations
+
+from contextlib import contextmanager
 
 import numpy as np
 import pytest
@@ -42,7 +47,18 @@ def _grid_operator(shape, extra=None):
     return row, c.astype(np.int32), np.where(r == c, diag[r], -1.0)
 
 
-def _check(row, col, val, nrhs, dtype, **opts):
+@contextmanager
+def resident(finished=0, declined=0, gave_up=0):
+    """The solves inside went to the resident engine this often, with these outcomes."""
+    from phipict_amd import profiling
+
+    before = profiling.resident_counts()
+    yield
+    got = tuple(b - a for a, b in zip(before, profiling.resident_counts()))
+    assert got == (finished, declined, gave_up), got
+
+
+def _check(row, col, val, nrhs, dtype, engine=dict(finished=1), **opts):
     import phipict_amd as pa
 
     n = row.size - 1
@@ -54,7 +70,8 @@ def _check(row, col, val, nrhs, dtype, **opts):
     A = pa.CSRmatrix(torch.as_tensor(val, dtype=tdt, device=DEV), torch.as_tensor(col, device=DEV),
                      torch.as_tensor(row, device=DEV))
     x = torch.as_tensor(x0.copy(), device=DEV)
-    infos = pa.SolveLinear(A, torch.as_tensor(b, device=DEV), x, maxIterations=4000, tolerance=tol, **opts)
+    with resident(**engine):
+        infos = pa.SolveLinear(A, torch.as_tensor(b, device=DEV), x, maxIterations=4000, tolerance=tol, **opts)
     xs = x.cpu().numpy().reshape(nrhs, n)
     for k in sorted({0, nrhs - 1}):
         xo = x0[k * n:(k + 1) * n].copy()
@@ -96,7 +113,8 @@ def test_residual_replacement_in_large_teams(shape):
 @pytest.mark.parametrize("n", [2000, 9000])
 def test_rows_beyond_the_kernels_take_another_engine(n):
     """One row of 13 entries among rows of five: no rows dropped."""
-    _check(*_grid_operator((n // 50, 50), extra=[(0, n - 1 - 7 * k) for k in range(10)]), 1, np.float64)
+    _check(*_grid_operator((n // 50, 50), extra=[(0, n - 1 - 7 * k) for k in range(10)]), 1, np.float64,
+           engine=dict(declined=1))
 
 
 @pytest.mark.parametrize("shapes,ncomp", [
@@ -120,8 +138,9 @@ def test_resident_segmented_cg_matches_oracle(shapes, ncomp):
     b[0, segs[1]:segs[2]] = 0.0  # a zero right-hand side: x = 0, no iterations
     A = pa.CSRmatrix(*(torch.as_tensor(a, device=DEV) for a in (val, col, row)))
     x = torch.as_tensor(x0.reshape(-1).copy(), device=DEV)
-    infos = pa.SolveSegmented(A, segs.tolist(), torch.as_tensor(b.reshape(-1), device=DEV), x, maxIterations=4000,
-                              tolerance=tol)
+    with resident(finished=1):
+        infos = pa.SolveSegmented(A, segs.tolist(), torch.as_tensor(b.reshape(-1), device=DEV), x, maxIterations=4000,
+                                  tolerance=tol)
     xs = x.cpu().numpy().reshape(ncomp, n)
     for c in range(ncomp):
         for s in range(S):
