@@ -420,6 +420,12 @@ int pp_solve_linear_noalloc(const pp_csr *A, const void *rhs, void *x, int32_t n
  * given-up solves were then run by the multi-launch engines. */
 int pp_resident_counts(int64_t *counts);
 
+/* Diagnostic (no reference counterpart): the polls a workgroup of the resident engine spends on one
+ * exchange before it gives up, for the solves of the calling host thread from now on: at most the
+ * built-in 2^21 (about two seconds), which a negative value restores. Small values make solves of
+ * several-workgroup teams give up, for tests of what happens then. */
+int pp_resident_wait(int32_t polls);
+
 /* replaces ReleaseKrylovWorkspaces (bindings.cpp:777, krylov.cu:921-924). */
 int pp_release_workspaces(void);
 

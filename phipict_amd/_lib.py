@@ -205,6 +205,7 @@ SIGNATURES = {
                          _i32, _i32, _i32, _i32, _i32, _dbl, _P(_dbl), _i32, _vp, _P(SolveResult)],
     "pp_release_workspaces": [],
     "pp_resident_counts": [_vp],
+    "pp_resident_wait": [_i32],
     "pp_sparse_outer_product": [_vp, _vp, _P(CsrDesc), _i32, _vp],
     "pp_csr_transpose": [_P(CsrDesc), _i32, _vp, _vp, _vp, _vp],
     "pp_spmv": [_P(CsrDesc), _vp, _vp, _i32, _i32, _vp],

@@ -20,9 +20,11 @@
 // all-gather and read the vector published with it. Without the all-gather at a replacement a member that
 // waits for its stencil neighbours' x alone would overwrite sums that a member farther away still polls.
 //
-// A team member that waits too long (RES_SPINS polls: some other process or a fault keeps a
-// workgroup of the team from running) gives up, and says so in the launch's `failed` word: the host then
-// runs the solve on the multi-launch engine. Teams are as large as the chip, not larger,
+// A team member that waits too long (some other process or a fault keeps a workgroup of the team from
+// running) gives up, and says so in the launch's `failed` word: the host then runs the solve on the
+// multi-launch engine. A thread spends RES_SPINS polls at most on the words of one vector and, in the
+// wave that folds, as many on the sums; polls left after a workgroup has given up anywhere in the launch
+// are not made, and a workgroup whose vector did not arrive does not wait for sums. Teams are as large as the chip, not larger,
 // and one launch of several-workgroup teams runs at a time per process (the host holds a lock), so
 // that all members are resident together.
 //
@@ -33,7 +35,6 @@
 namespace pp {
 
 typedef unsigned long long word_t;
-constexpr int RES_SPINS = 1 << 21;
 constexpr int RES_WAVES = 16;
 constexpr int RES_POLL = 2; // members a lane of the deciding wave polls at a time
 
@@ -80,6 +81,7 @@ struct Team {
     word_t *slots;       // [2][3][wgs] tagged doubles
     int wg, wg0, G, wgs; // this workgroup, the team's first, their number, all workgroups of the launch
     unsigned tag;        // of the latest exchange
+    Patience fresh;      // what a wait starts with
 };
 // What wave 0 tells the workgroup after a decision.
 struct Verdict {
@@ -90,7 +92,9 @@ struct TeamLds {
     double part[3][RES_WAVES]; // per wave: this workgroup's sums
     SolveRec S;
     Verdict out;
-    int bad; // a poll gave up
+    int bad;  // a word of a vector did not arrive
+    int quit; // as of the latest decision: `bad`, or sums that did not arrive (written by the first wave
+              // between the barriers of a decision, so that all threads read the same)
 };
 
 // The team's totals of v[q], handed to `decide` in wave 0 (all its lanes hold them, the same bits in
@@ -123,10 +127,11 @@ __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], Tea
             double got[NQ];
 #pragma unroll
             for (int q = 0; q < NQ; ++q) got[q] = 0.0;
-            bool late = false;
+            bool late = L.bad != 0;
+            Patience left = tm.fresh;
+            if (late) left.left = 0;
             for (int g0 = 0; g0 < tm.G; g0 += 64 * RES_POLL) {
                 Tagged<double> m[RES_POLL][NQ];
-                int spins = 0;
                 bool ok;
                 do {
                     ok = true;
@@ -141,7 +146,7 @@ __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], Tea
 #pragma unroll
                         for (int q = 0; q < NQ; ++q)
                             if (g0 + 64 * u + t < tm.G) ok = ok && m[u][q].is(tm.tag);
-                } while (!ok && ++spins < RES_SPINS);
+                } while (!ok && left.more());
                 late = late || !ok;
 #pragma unroll
                 for (int u = 0; u < RES_POLL; ++u)
@@ -149,7 +154,7 @@ __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], Tea
                     for (int q = 0; q < NQ; ++q)
                         if (g0 + 64 * u + t < tm.G) got[q] += m[u][q].value();
             }
-            if (late) L.bad = 1;
+            if (late) L.quit = 1;
 #pragma unroll
             for (int q = 0; q < NQ; ++q) tot[q] = wave_total(got[q]);
         }
@@ -162,7 +167,7 @@ __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], Tea
         }
     }
     __syncthreads();
-    return LOCAL || L.bad == 0;
+    return LOCAL || L.quit == 0;
 }
 template <int NQ, bool LOCAL, typename F>
 __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], TeamLds &L, F decide) {
@@ -280,8 +285,9 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     const Share sh = share_of(a, tm, blk * R);
     tm.slots = a.slots;
     tm.tag = a.tag;
+    tm.fresh = Patience{a.spins, a.failed, a.done};
     if (t == 0) {
-        L.bad = 0;
+        L.bad = L.quit = 0;
         L.S = rec_init(tol_of(a, sh.piece), a.maxit);
         L.out = Verdict{0.0, 1, 1, 0, 0};
     }
@@ -322,7 +328,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     };
     // the values published under `tag` for the entries of row k (the codes pass through `hide`, so
     // that no address derived from them is kept in registers over the iterations)
-    auto gather = [&](int k, unsigned tag, T (&out)[EW]) {
+    auto gather = [&](int k, unsigned tag, T (&out)[EW], Patience &left) {
         Tagged<T> g[EW];
         int c[EW];
         const word_t *Z = zpar(tag) + ((size_t)sh.vbase - a.zorigin) * TW;
@@ -335,8 +341,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
         for (int j = 0; j < EW; ++j) {
             if (LOCAL || c[j] >= 0) out[j] = zs[c[j]];
             else {
-                int spins = 0;
-                while (!g[j].is(tag) && ++spins < RES_SPINS) g[j].load(Z + unsigned(-1 - c[j]) * TW);
+                while (!g[j].is(tag) && left.more()) g[j].load(Z + unsigned(-1 - c[j]) * TW);
                 if (!g[j].is(tag)) L.bad = 1;
                 out[j] = g[j].value();
             }
@@ -347,9 +352,11 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     constexpr bool EARLY = !LOCAL && R <= 2;
     T zn[EARLY ? R : 1][EW];
     auto fetch = [&] {
-        if constexpr (EARLY)
+        if constexpr (EARLY) {
+            Patience left = tm.fresh;
 #pragma unroll
-            for (int k = 0; k < R; ++k) gather(k, tm.tag, zn[k]);
+            for (int k = 0; k < R; ++k) gather(k, tm.tag, zn[k], left);
+        }
     };
     {
         // r = b - A x
@@ -408,12 +415,13 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
             const double none[1] = {0.0};
             if (!team_decide<1, LOCAL>(tm, none, L, [](const double (&)[1], SolveRec &, Verdict &) {})) return give_up(a);
             const unsigned xtag = tm.tag;
+            Patience left = tm.fresh;
             double s[2] = {0.0, 0.0};
             T z[R];
 #pragma unroll
             for (int k = 0; k < R; ++k) {
                 T xn[EW], ax = T(0);
-                gather(k, xtag, xn);
+                gather(k, xtag, xn, left);
 #pragma unroll
                 for (int j = 0; j < EW; ++j) ax += M.a[k][j] * xn[j];
                 if (t + k * blk < own) r[k] = rhs(k) - ax;
@@ -451,10 +459,11 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
             }
         } else {
             // p' = z + beta p at every neighbour as its z arrives, q = A p'
+            Patience left = tm.fresh;
 #pragma unroll
             for (int k = 0; k < R; ++k) {
                 T zk[EW], s = T(0);
-                if constexpr (!EARLY) gather(k, ztag, zk);
+                if constexpr (!EARLY) gather(k, ztag, zk, left);
 #pragma unroll
                 for (int j = 0; j < EW; ++j) {
                     const T z = EARLY ? zn[k][j] : zk[j];

@@ -4,12 +4,14 @@
 #pragma once
 
 #include "pp_krylov.hpp"
+#include "pp_patience.hpp"
 
 namespace pp {
 
 constexpr int RES_WG = 512;        // threads of a multi-workgroup team's workgroups
 constexpr int RES_LOCAL_WG = 1024; // threads at most of a one-workgroup team
 constexpr int RES_TOLS = 8;        // tolerances passed by value
+constexpr int RES_SPINS = 1 << 21; // polls a thread spends on one exchange before it gives up, about a microsecond each
 
 // Pieces of a segmented solve: piece k has len[k] rows at vector offset base[k], its matrix rows
 // start at mrow[k]; workgroup w of the launch works on piece wgPiece[w], whose workgroups are
@@ -33,6 +35,7 @@ struct ResArgs {
     unsigned *failed;            // `done` from a workgroup that gave up waiting
     unsigned *declined;          // `done` from a workgroup whose team has a row longer than the kernel takes
     unsigned tag, done;          // the exchanges' first tag less one; the launch's word
+    int spins;                   // RES_SPINS, less where a test wants teams to give up
     int n, rpm, G, team0;        // plain solve: rows, right-hand sides per matrix, workgroups per team, first team
     int wgs;                     // workgroups of the launch
     int maxit, returnBest, project, resetEvery;

@@ -1176,6 +1176,7 @@ struct ThreadSpaces {
     void *tbuf = nullptr; size_t tcap = 0;
     int *tbad = nullptr;
     int64_t resident[3] = {0, 0, 0}; // solves the resident engine finished, declined and gave up on
+    int residentSpins = RES_SPINS;
 };
 static std::vector<ThreadSpaces *> g_all_spaces; // every thread's, for pp_release_workspaces
 
@@ -1731,6 +1732,7 @@ static void resident_status(Space &sp, int B, ResArgs<T> *a) {
     a->failed = a->status + B;
     a->declined = a->status + B + 1;
     a->done = 0xC0DE0000u + (++sp.solves & 0xffffu);
+    a->spins = my_spaces().residentSpins;
 }
 
 // All of it back in one copy; *ran: every team finished (counted, with the ways it can fail, for the
@@ -3002,6 +3004,11 @@ int pp_amg_pcg_solve(const pp_csr *A, const pp_amg_level *levels, int32_t num_le
 int pp_resident_counts(int64_t *counts) {
     PP_CHECK_ARG(counts, "null argument");
     for (int k = 0; k < 3; ++k) counts[k] = my_spaces().resident[k];
+    return PP_OK;
+}
+
+int pp_resident_wait(int32_t polls) {
+    my_spaces().residentSpins = polls < 0 ? RES_SPINS : std::min<int>(polls, RES_SPINS);
     return PP_OK;
 }
 

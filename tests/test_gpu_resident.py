@@ -110,6 +110,27 @@ def test_residual_replacement_in_large_teams(shape):
     _check(*_grid_operator(shape), 1, np.float64, residualResetSteps=7)
 
 
+@contextmanager
+def no_waiting():
+    """Teams of several workgroups give up at the first word that is not there yet."""
+    from phipict_amd import _lib
+
+    _lib.call("pp_resident_wait", 0)
+    try:
+        yield
+    finally:
+        _lib.call("pp_resident_wait", -1)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("shape,nrhs", [((65, 64), 3), ((200, 190), 2), ((331, 396), 1), ((20, 31, 33), 2), ((71, 60, 62), 1)])
+def test_given_up_solves_are_run_by_the_other_engines(shape, nrhs, dtype):
+    """Rows up to 32768: the one-workgroup engine; above: a launch per phase."""
+    print(f"[resident] giving up {shape} x {nrhs} {np.dtype(dtype).name}", flush=True)
+    with no_waiting():
+        _check(*_grid_operator(shape), nrhs, dtype, engine=dict(gave_up=1))
+
+
 @pytest.mark.parametrize("n", [2000, 9000])
 def test_rows_beyond_the_kernels_take_another_engine(n):
     """One row of 13 entries among rows of five: no rows dropped."""
