@@ -32,6 +32,8 @@
 // applies them to its own copy of the record, from sums folded in one fixed order by every workgroup.
 #include "pp_resident.hpp"
 
+#include <algorithm>
+
 namespace pp {
 
 typedef unsigned long long word_t;
@@ -268,9 +270,21 @@ template <typename T>
 __device__ __forceinline__ void give_up(const ResArgs<T> &a) {
     if (threadIdx.x == 0) *a.failed = a.done;
 }
-template <typename T>
-__device__ __forceinline__ void decline(const ResArgs<T> &a) {
-    if (threadIdx.x == 0) *a.declined = a.done;
+
+// Rows longer than the resident kernels take. They are looked for before anything is solved: pieces that
+// found one in their own rows while the others solved theirs would leave x half done for the engine
+// that takes over. Right-hand sides of one workgroup each look for themselves (they share the pattern, so
+// all of them find it): the launch takes 4 us, the solve of 4 k rows 900.
+__global__ void __launch_bounds__(256) k_row_check(const int32_t *__restrict__ row, int n, int ew, unsigned *declined,
+                                                   unsigned word) {
+    bool lng = false;
+    for (int i = blockIdx.x * 256 + (int)threadIdx.x; i < n; i += gridDim.x * 256) lng |= row[i + 1] - row[i] > ew;
+    if (lng) *declined = word;
+}
+int launch_row_check(const int32_t *row, int n, int ew, unsigned *declined, unsigned word, hipStream_t s) {
+    hipLaunchKernelGGL(k_row_check, dim3(std::min(512, (n + 255) / 256)), dim3(256), 0, s, row, n, ew, declined, word);
+    PP_LAUNCH_CHECK();
+    return PP_OK;
 }
 
 // CG (with dinv its Jacobi variant), a team per right-hand side.
@@ -281,6 +295,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     T *zs = reinterpret_cast<T *>(res_lds); // exchanged values of the workgroup's own rows
     __shared__ TeamLds L;
     const int t = threadIdx.x, blk = blockDim.x;
+    if (*a.declined == a.done) return;
     Team tm;
     const Share sh = share_of(a, tm, blk * R);
     tm.slots = a.slots;
@@ -293,26 +308,28 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     }
     Rows<T, EW, R> M;
     const bool fits = M.load(a.A, sh);
+    if constexpr (LOCAL)
+        if (__syncthreads_or(!fits)) {
+            if (t == 0) *a.declined = a.done;
+            return;
+        }
     const T *dv = a.dinv ? a.dinv + (size_t)sh.m * a.dinvStride + sh.row0 : nullptr;
     const int own = sh.n - sh.row0; // rows k with t + k * blk < own belong to this thread
     const size_t v0 = (size_t)sh.vbase + sh.row0 + t; // vector offset of the thread's first row
     T x[R], r[R], p[R];
     T mean = T(0);
     __syncthreads();
-    {
-        // rows that do not fit, and the mean of b to project out
-        double s[2] = {fits ? 0.0 : 1.0, 0.0};
-        if (a.project)
+    if (a.project) {
+        // the mean of b
+        double s[1] = {0.0};
 #pragma unroll
-            for (int k = 0; k < R; ++k)
-                if (t + k * blk < own) s[1] += double(a.b[v0 + k * blk]);
-        if (!team_decide<2, LOCAL>(tm, s, L, [&](const double (&tot)[2], SolveRec &, Verdict &o) {
-                o.active = tot[0] == 0.0;
-                o.step = tot[1] / double(sh.n);
+        for (int k = 0; k < R; ++k)
+            if (t + k * blk < own) s[0] += double(a.b[v0 + k * blk]);
+        if (!team_decide<1, LOCAL>(tm, s, L, [&](const double (&tot)[1], SolveRec &, Verdict &o) {
+                o.step = tot[0] / double(sh.n);
             }))
             return give_up(a);
-        if (!L.out.active) return decline(a);
-        if (a.project) mean = T(L.out.step);
+        mean = T(L.out.step);
     }
     auto rhs = [&](int k) { return a.project ? a.b[v0 + k * blk] - mean : a.b[v0 + k * blk]; };
     auto zof = [&](int k) { return dv && t + k * blk < own ? r[k] * dv[t + k * blk] : r[k]; };

@@ -33,7 +33,7 @@ struct ResArgs {
     SolveRec *recs;              // final records
     unsigned *status;            // per right-hand side: `done` from the team that finished it
     unsigned *failed;            // `done` from a workgroup that gave up waiting
-    unsigned *declined;          // `done` from a workgroup whose team has a row longer than the kernel takes
+    unsigned *declined;          // `done`: a row is longer than the kernel takes, nothing is solved
     unsigned tag, done;          // the exchanges' first tag less one; the launch's word
     int spins;                   // RES_SPINS, less where a test wants teams to give up
     int n, rpm, G, team0;        // plain solve: rows, right-hand sides per matrix, workgroups per team, first team
@@ -49,6 +49,9 @@ struct ResArgs {
 
 // Largest one-workgroup system, in rows, for stencil rows of `ew` entries.
 inline int resident_local_rows(int ew) { return (ew == 5 ? 4 : 3) * RES_LOCAL_WG; }
+
+// *declined = word if one of the n CSR rows has more than ew entries; run before the launches that look at it.
+int launch_row_check(const int32_t *row, int n, int ew, unsigned *declined, unsigned word, hipStream_t s);
 
 // Launch on `wgs` workgroups: local = every team is one workgroup of `threads` threads with up
 // to R rows per thread; otherwise teams of RES_WG-thread workgroups with R rows per thread.

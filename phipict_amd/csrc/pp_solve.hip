@@ -1668,7 +1668,7 @@ struct ResPlan {
 };
 
 // Entries per row the kernels are built for: the ELL width, or for plain CSR a guess from the
-// mean row length, which the kernel checks against every row.
+// mean row length, checked against every row before the solve.
 template <typename T>
 static int resident_width(const Csr<T> &A, long nnz) {
     if (A.ell_w > 0) return A.ell_w == 5 || A.ell_w == 7 ? A.ell_w : 0;
@@ -1724,15 +1724,16 @@ static uint32_t resident_tags(int maxit) { return (uint32_t)(4 * ((int64_t)maxit
 
 // Where a resident solve of B right-hand sides leaves its records, then (in the second record copy's
 // place) a word per team, one for teams that gave up and one for teams that declined, told from older
-// contents by this solve's value.
+// contents by this solve's value. check: looks for CSR rows longer than the `ew` entries of the kernels.
 template <typename T>
-static void resident_status(Space &sp, int B, ResArgs<T> *a) {
+static int resident_status(Space &sp, int B, int ew, bool check, hipStream_t s, ResArgs<T> *a) {
     a->recs = recs_a(sp);
     a->status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
     a->failed = a->status + B;
     a->declined = a->status + B + 1;
     a->done = 0xC0DE0000u + (++sp.solves & 0xffffu);
     a->spins = my_spaces().residentSpins;
+    return !check || a->A.ell_w > 0 ? PP_OK : launch_row_check(a->A.row, a->A.n, ew, a->declined, a->done, s);
 }
 
 // All of it back in one copy; *ran: every team finished (counted, with the ways it can fail, for the
@@ -1788,7 +1789,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
         a.slots = a.zbuf + zWords;
         a.tag = tag;
     }
-    resident_status(sp, B, &a);
+    if (int e = resident_status(sp, B, plan.ew, !plan.local, s, &a)) return e;
     for (int t0 = 0; t0 < B; t0 += plan.perLaunch) {
         const int teams = std::min(plan.perLaunch, B - t0);
         a.team0 = t0;
@@ -2656,7 +2657,7 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
         a.slots = a.zbuf + zWords;
         a.tag = tag;
     }
-    resident_status(sp, K, &a);
+    if (int e = resident_status(sp, K, ew, true, s, &a)) return e;
     for (int l = 0; l < pack.launches + (pack.localR ? 1 : 0); ++l) {
         const bool local = l == pack.launches;
         a.wgs = (local ? (int)pack.wgPiece.size() : pack.wgFirst[l + 1]) - pack.wgFirst[l];

@@ -75,7 +75,7 @@ def member(me, sums, vecs, needs, iterations, reset_every, early, sound):
                 yield
             yield
 
-    yield from all_gather()                      # row check, mean of b
+    yield from all_gather()                      # mean of b
     yield from publish()                         # z
     yield from all_gather(needs if early else ())
     ztag = tag

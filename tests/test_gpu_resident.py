@@ -138,6 +138,42 @@ def test_rows_beyond_the_kernels_take_another_engine(n):
            engine=dict(declined=1))
 
 
+def _segmented(parts, segs):
+    import phipict_amd as pa
+
+    offs = np.concatenate([[0], np.cumsum([p[1].size for p in parts])])
+    row = np.concatenate([[0]] + [p[0][1:] + off for p, off in zip(parts, offs)]).astype(np.int32)
+    col = np.concatenate([p[1] + o for p, o in zip(parts, segs)]).astype(np.int32)
+    val = np.concatenate([p[2] for p in parts])
+    return pa.CSRmatrix(*(torch.as_tensor(a, device=DEV) for a in (val, col, row)))
+
+
+def _solve_pieces_from_the_start_guess(parts, engine):
+    """Every piece is solved once, from the caller's start guess: the oracle's iterations."""
+    import phipict_amd as pa
+
+    segs = np.concatenate([[0], np.cumsum([p[0].size - 1 for p in parts])])
+    rng = np.random.default_rng(12)
+    b, x0 = rng.standard_normal(segs[-1]), 0.1 * rng.standard_normal(segs[-1])
+    x = torch.as_tensor(x0.copy(), device=DEV)
+    with resident(**engine):
+        infos = pa.SolveSegmented(_segmented(parts, segs), segs.tolist(), torch.as_tensor(b, device=DEV), x,
+                                  maxIterations=4000, tolerance=1e-9)
+    xs = x.cpu().numpy()
+    for k, (lo, hi) in enumerate(zip(segs[:-1], segs[1:])):
+        xo = x0[lo:hi].copy()
+        ref = O.cg(*parts[k], b[lo:hi].copy(), xo, 1e-9, maxit=4000)
+        assert infos[k].converged and abs(infos[k].usedIterations - ref.used_iterations) <= 1, (k, infos[k], ref)
+        assert np.linalg.norm(xs[lo:hi] - xo) <= 2 * np.sqrt(hi - lo) * 1e-9 / SHIFT + 1e-14 * np.linalg.norm(xo)
+
+
+def test_one_long_row_leaves_no_piece_half_solved():
+    """A piece with a row of 13 entries among pieces of five: declined before any piece is solved."""
+    _solve_pieces_from_the_start_guess([_grid_operator((20, 31)), _grid_operator((70, 65)), _grid_operator((9, 40)),
+                                        _grid_operator((30, 20), extra=[(0, 599 - 7 * k) for k in range(10)])],
+                                       dict(declined=1))
+
+
 @pytest.mark.parametrize("shapes,ncomp", [
     ([(9, 7), (64, 64), (30, 2)], 2),                     # one workgroup each
     ([(65, 64), (20, 11), (300, 220), (3, 3)], 1),        # teams, the small ones beside them
