@@ -21,6 +21,7 @@
 #include "pp_resident.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -1153,7 +1154,6 @@ struct Space {
     char *snap = nullptr;  size_t snapCap = 0;  // pinned snapshots: two slots of B records
     void *link = nullptr;  size_t linkCap = 0;  // tagged words of the resident engine, never anything else
     uint32_t linkTag = 0;                       // the largest tag they may hold
-    unsigned solves = 0;                        // resident solves so far: their status word
     bool fixed = false;    // carved from the static scratch array: never grows, never freed
     hipEvent_t ev[2] = {nullptr, nullptr}; // snapshot events created once (fixed spaces)
 };
@@ -1724,14 +1724,16 @@ static uint32_t resident_tags(int maxit) { return (uint32_t)(4 * ((int64_t)maxit
 
 // Where a resident solve of B right-hand sides leaves its records, then (in the second record copy's
 // place) a word per team, one for teams that gave up and one for teams that declined, told from older
-// contents by this solve's value. check: looks for CSR rows longer than the `ew` entries of the kernels.
+// contents (records, or words of solves before, also in memory released and allocated again) by
+// this solve's value. check: looks for CSR rows longer than the `ew` entries of the kernels.
+static std::atomic<unsigned> g_resident_solves{0}; // of all threads
 template <typename T>
 static int resident_status(Space &sp, int B, int ew, bool check, hipStream_t s, ResArgs<T> *a) {
     a->recs = recs_a(sp);
     a->status = reinterpret_cast<unsigned *>(recs_a(sp) + B);
     a->failed = a->status + B;
     a->declined = a->status + B + 1;
-    a->done = 0xC0DE0000u + (++sp.solves & 0xffffu);
+    a->done = 0x9E3779B1u * ++g_resident_solves;
     a->spins = my_spaces().residentSpins;
     return !check || a->A.ell_w > 0 ? PP_OK : launch_row_check(a->A.row, a->A.n, ew, a->declined, a->done, s);
 }

@@ -138,6 +138,18 @@ def test_rows_beyond_the_kernels_take_another_engine(n):
            engine=dict(declined=1))
 
 
+def test_a_declined_solve_leaves_nothing_behind():
+    """The words by which a launch reports are not taken for those of a solve before, also where the workspace
+    was released and its memory comes back as it was."""
+    import phipict_amd as pa
+
+    for shape in ((40, 50), (180, 50)):
+        pa.ReleaseKrylovWorkspaces()
+        _check(*_grid_operator(shape, extra=[(0, 1990 - 7 * k) for k in range(10)]), 1, np.float64, engine=dict(declined=1))
+        pa.ReleaseKrylovWorkspaces()
+        _check(*_grid_operator(shape), 1, np.float64)
+
+
 def _segmented(parts, segs):
     import phipict_amd as pa
 
