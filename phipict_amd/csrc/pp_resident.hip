@@ -21,8 +21,8 @@
 // waits for its stencil neighbours' x alone would overwrite sums that a member farther away still polls.
 //
 // A team member that waits too long (some other process or a fault keeps a workgroup of the team from
-// running) gives up, and says so in the launch's `failed` word: the host then runs the solve on the
-// multi-launch engine. A thread spends RES_SPINS polls at most on the words of one vector and, in the
+// running) gives up, and says so in the launch's `failed` word: the host then puts the start guess back,
+// which teams that finished have overwritten, and runs the solve on the multi-launch engine. A thread spends RES_SPINS polls at most on the words of one vector and, in the
 // wave that folds, as many on the sums; polls left after a workgroup has given up anywhere in the launch
 // are not made, and a workgroup whose vector did not arrive does not wait for sums. Teams are as large as the chip, not larger,
 // and one launch of several-workgroup teams runs at a time per process (the host holds a lock), so
@@ -317,6 +317,11 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     const int own = sh.n - sh.row0; // rows k with t + k * blk < own belong to this thread
     const size_t v0 = (size_t)sh.vbase + sh.row0 + t; // vector offset of the thread's first row
     T x[R], r[R], p[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        x[k] = T(0);
+        if (t + k * blk < own) a.x0[v0 + k * blk] = x[k] = a.x[v0 + k * blk];
+    }
     T mean = T(0);
     __syncthreads();
     if (a.project) {
@@ -382,7 +387,6 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             const bool in = t + k * blk < own;
-            x[k] = in ? a.x[v0 + k * blk] : T(0);
             p[k] = r[k] = T(0);
             if (in) {
                 T ax = T(0);

@@ -25,6 +25,7 @@ struct ResArgs {
     Csr<T> A;
     const T *b;
     T *x, *xbest;                // xbest: null without return-best
+    T *x0;                       // gets the start guess, for the host to put back when a team gave up
     const T *dinv;               // Jacobi preconditioner (null: none)
     int dinvStride;
     unsigned long long *zbuf;    // exchanged vectors: [2][vecLen] values in tagged words

@@ -1739,9 +1739,10 @@ static int resident_status(Space &sp, int B, int ew, bool check, hipStream_t s, 
 }
 
 // All of it back in one copy; *ran: every team finished (counted, with the ways it can fail, for the
-// calling thread).
+// calling thread). Otherwise the `len` values of x are the start guess again: teams that finished
+// beside one that gave up have written theirs, and the engine that takes over is not to start from those.
 template <typename T>
-static int resident_results(Space &sp, int B, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran) {
+static int resident_results(Space &sp, int B, size_t len, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran) {
     PP_HIP(hipMemcpyAsync(sp.snap, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 2), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     *recs = reinterpret_cast<const SolveRec *>(sp.snap);
@@ -1750,10 +1751,14 @@ static int resident_results(Space &sp, int B, const ResArgs<T> &a, hipStream_t s
     *ran = st[B] != a.done && !declined;
     for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
     ++my_spaces().resident[*ran ? 0 : (declined ? 1 : 2)];
+    if (!*ran && !declined) {
+        PP_HIP(hipMemcpyAsync(a.x, a.x0, sizeof(T) * len, hipMemcpyDeviceToDevice, s));
+        PP_HIP(hipStreamSynchronize(s)); // x0 lies in a workspace that the next engine may grow
+    }
     return PP_OK;
 }
 
-// *ran: the engine finished the solve (false: run another engine; x holds a start guess).
+// *ran: the engine finished the solve (false: run another engine; x holds the start guess).
 template <typename T>
 static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x, int B, int maxit, const double *tols,
                           int ntols, double scale, int resetEvery, int returnBest, int project, int bicg, int jacobi,
@@ -1762,13 +1767,13 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
     *ran = false;
     const int numMat = (B + A.rpm - 1) / A.rpm;
     const size_t len = (size_t)n * B;
-    if (int e = prepare(sp, sizeof(T) * (len + (size_t)numMat * n), 8, B, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
+    if (int e = prepare(sp, sizeof(T) * (2 * len + (size_t)numMat * n), 8, B, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
     T *xbest = reinterpret_cast<T *>(sp.vec);
-    T *dinv = jacobi ? xbest + len : nullptr;
+    T *dinv = jacobi ? xbest + 2 * len : nullptr;
     if (jacobi) launch_jacobi<T>(A, numMat, dinv, s);
     ResArgs<T> a{};
     a.A = A;
-    a.b = b; a.x = x; a.xbest = returnBest ? xbest : nullptr;
+    a.b = b; a.x = x; a.xbest = returnBest ? xbest : nullptr; a.x0 = xbest + len;
     a.dinv = dinv; a.dinvStride = A.valStride ? n : 0;
     a.vecLen = (size_t)n * plan.perLaunch;
     a.n = n; a.rpm = A.rpm; a.G = plan.G;
@@ -1804,7 +1809,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
         a.tag += tags;
         sp.linkTag += plan.local ? 0 : tags;
     }
-    return resident_results(sp, B, a, s, recs, ran);
+    return resident_results(sp, B, len, a, s, recs, ran);
 }
 
 // ---------------- small systems ----------------
@@ -2634,7 +2639,8 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
     if ((uint64_t)tags * std::max(1, pack.launches) > (1u << 31)) return PP_OK;
     SegSpace &sg = my_spaces().seg;
     Space &sp = sg.sp;
-    if (int e = prepare(sp, 256, 8, K, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
+    const size_t total = (size_t)ncomp * N;
+    if (int e = prepare(sp, sizeof(T) * total, 8, K, tols, ntols > RES_TOLS ? ntols : 0, s)) return e;
     // the layout: base len mrow wg0 G [K], wgPiece, through a pinned staging copy (rewritten only after
     // this solve's final wait)
     std::vector<int32_t> host;
@@ -2643,8 +2649,8 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
     const int32_t *ld = sg.layoutDev;
     ResArgs<T> a{};
     a.A = A;
-    a.b = b; a.x = x;
-    a.vecLen = (size_t)ncomp * N;
+    a.b = b; a.x = x; a.x0 = reinterpret_cast<T *>(sp.vec);
+    a.vecLen = total;
     a.maxit = maxit; a.project = project; a.zeroStops = 1;
     a.ntols = ntols > RES_TOLS ? 1 : ntols;
     for (int k = 0; k < a.ntols; ++k) a.tols[k] = tols[k];
@@ -2672,7 +2678,7 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
         if (!local) sp.linkTag += tags;
     }
     const SolveRec *recs = nullptr;
-    if (int e = resident_results(sp, K, a, s, &recs, ran)) return e;
+    if (int e = resident_results(sp, K, total, a, s, &recs, ran)) return e;
     if (!*ran) return PP_OK;
     report(recs, K, 0, res);
     for (int k = 0; k < K; ++k)

@@ -179,6 +179,14 @@ def _solve_pieces_from_the_start_guess(parts, engine):
         assert np.linalg.norm(xs[lo:hi] - xo) <= 2 * np.sqrt(hi - lo) * 1e-9 / SHIFT + 1e-14 * np.linalg.norm(xo)
 
 
+def test_giving_up_leaves_no_piece_half_solved():
+    """The piece of several workgroups gives up, those of one workgroup beside it finish: all solved from the
+    start guess."""
+    with no_waiting():
+        _solve_pieces_from_the_start_guess([_grid_operator((20, 31)), _grid_operator((70, 65)), _grid_operator((9, 40))],
+                                           dict(gave_up=1))
+
+
 def test_one_long_row_leaves_no_piece_half_solved():
     """A piece with a row of 13 entries among pieces of five: declined before any piece is solved."""
     _solve_pieces_from_the_start_guess([_grid_operator((20, 31)), _grid_operator((70, 65)), _grid_operator((9, 40)),
