@@ -403,7 +403,7 @@ int pp_solve_segmented(const pp_csr *A, const int32_t *seg_rows, int32_t nseg, i
 /* No counterpart in the reference: pp_solve_linear for callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). Same
  * arguments, results and kernels as pp_solve_linear, but every work buffer (vectors, partial
- * sums, solve records, tolerances, exchanged words) comes from one static device array of 83.1 MiB
+ * sums, solve records, tolerances, exchanged words) comes from one static device array of 79.1 MiB
  * per GPU (56 MiB of work vectors: e.g. seven vectors of 1.0 M doubles), the host snapshots from a static
  * host array (at most 2048 right-hand sides) and the snapshot events are created at the first
  * call on a device; it calls no hipMalloc, hipFree or other allocating routine. Larger solves

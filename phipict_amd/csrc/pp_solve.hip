@@ -1522,6 +1522,14 @@ static void launch_jacobi(const Csr<T> &A, int numMat, T *dv, hipStream_t s) {
 }
 
 // ---------------- CG (large systems) ----------------
+constexpr int CG_LARGE_VECS = 6, CG_LARGE_PARTS = 1 + 3 + 1 + 2; // vectors and partial sets per right-hand side
+// Grid rows (each up to four right-hand sides of one matrix) and workgroups of each.
+static void cg_large_grid(int n, int B, int rpm, int *rows, int *G) {
+    const int NBv = std::min(rpm, 4);
+    *rows = (B + rpm - 1) / rpm * ((rpm + NBv - 1) / NBv);
+    *G = phase_width(n, *rows, WG);
+}
+
 template <typename T>
 static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const double *tols, int ntols, double scale,
                     int resetEvery, int returnBest, int project, int jacobi, Space &sp, hipStream_t s,
@@ -1529,11 +1537,12 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
     const int n = A.n;
     const int NBv = std::min(A.rpm, 4);
     const int numMat = (B + A.rpm - 1) / A.rpm;
-    const int rows = numMat * ((A.rpm + NBv - 1) / NBv);
-    const int G = phase_width(n, rows, WG);
+    int rows, G;
+    cg_large_grid(n, B, A.rpm, &rows, &G);
     enum { V_R = 0, V_Q, V_P0, V_P1, V_XB, V_BW, V_COUNT };
+    static_assert(V_COUNT == CG_LARGE_VECS);
     const size_t vecBytes = sizeof(T) * ((size_t)V_COUNT * n * B + (size_t)numMat * n);
-    const size_t partDoubles = (size_t)B * G * (1 + 3 + 1 + 2);
+    const size_t partDoubles = (size_t)B * G * CG_LARGE_PARTS;
     if (int e = prepare(sp, vecBytes, partDoubles, B, tols, ntols, s)) return e;
     T *vec = reinterpret_cast<T *>(sp.vec);
     auto V = [&](int k) { return vec + (size_t)k * n * B; };
@@ -1702,10 +1711,10 @@ static ResPlan resident_plan(int n, int teams, int ew) {
     return p;
 }
 
-// `words` tagged words whose tags are at most *tag, with room for `tags` more.
+// `words` tagged words (of which a fixed space holds enough) whose tags are at most *tag, with room for
+// `tags` more.
 static int resident_link(Space &sp, size_t words, uint32_t tags, hipStream_t s, uint32_t *tag) {
     const size_t bytes = words * sizeof(uint64_t);
-    if (sp.fixed) PP_CHECK_ARG(bytes <= sp.linkCap, "solve exceeds the static exchange buffer");
     const bool grown = sp.linkCap < bytes;
     if (int e = grown ? grow(&sp.link, &sp.linkCap, bytes) : PP_OK) return e;
     if (grown || sp.linkTag > UINT32_MAX - tags) {
@@ -1787,6 +1796,7 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
     const uint32_t tags = resident_tags(maxit);
     const int launches = (B + plan.perLaunch - 1) / plan.perLaunch;
     if (!plan.local && (uint64_t)tags * launches > (1u << 31)) return PP_OK;
+    if (sp.fixed && (zWords + slotWords) * sizeof(uint64_t) > sp.linkCap) return PP_OK;
     std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
     if (!plan.local) alone.lock();
     if (!plan.local) {
@@ -2817,6 +2827,15 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
         if (plan.ew && maxit <= RES_MAXIT && (small || plan.perLaunch >= nrhs)) {
             const SolveRec *recs = nullptr;
             bool ran = false;
+            if (sp.fixed) {
+                // taken only if the engine behind it fits the static scratch too, which has to solve it if a
+                // team gives up
+                int rows, G;
+                cg_large_grid(A->n, nrhs, rpm, &rows, &G);
+                const size_t vecs = (size_t)(small ? SMALL_SLOTS : CG_LARGE_VECS) * A->n * nrhs + (size_t)A->num_matrices * A->n;
+                if (int e = prepare(sp, sizeof(T) * vecs, small ? 8 : (size_t)nrhs * G * CG_LARGE_PARTS, nrhs, tols, ntols, s))
+                    return e;
+            }
             if (int e = resident_solve<T>(C, plan, b, xx, nrhs, maxit, tols, ntols, scale,
                                           use_bicg ? 0 : residual_reset_steps, return_best, matrix_rank_deficient, use_bicg,
                                           jacobi, !small && nrhs == 1, sp, s, &recs, &ran))
@@ -2852,7 +2871,9 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
 // array and the snapshot events are created at that set-up too.
 constexpr size_t SCR_VEC = size_t(56) << 20, SCR_PARTS = size_t(6) << 20, SCR_RECS = size_t(1) << 20,
                  SCR_TOLS = size_t(64) << 10;
-constexpr size_t SCR_LINK = size_t(20) << 20; // tagged words of the resident engine: 262144 doubles and their sums
+// tagged words of the resident engine: the doubles (two words each, two parities) of the largest plan on
+// 256 CUs, four rows per thread, and 64 KiB of sums
+constexpr size_t SCR_LINK = size_t(256) * 4 * RES_WG * 32 + (size_t(64) << 10);
 constexpr size_t SCRATCH_BYTES = SCR_VEC + SCR_PARTS + SCR_RECS + SCR_TOLS + SCR_LINK;
 constexpr int SCRATCH_RHS = 2048;     // right-hand sides per call at most
 constexpr int SCRATCH_DEVICES = 16;   // devices of one process with a scratch table entry

@@ -96,3 +96,42 @@ def test_noalloc_refuses_beyond_scratch():
     msg.restype = C.c_char_p
     assert b"scratch maximum" in msg()
     assert float(x.abs().max()) == 0.0  # nothing ran
+
+
+def _grid_case(nx, ny, nrhs):
+    row, col, val = _poisson(nx, ny, 0.5)
+    t = [torch.as_tensor(a, device=DEV) for a in (row, col, val)]
+    b = torch.as_tensor(np.random.default_rng(ny).standard_normal(nrhs * nx * ny), device=DEV)
+    return t, b, torch.zeros_like(b)
+
+
+@pytest.mark.parametrize("nrhs,fits", [(203, True), (204, False)])
+def test_noalloc_batches_are_refused_by_the_engine_behind(nrhs, fits):
+    """Right-hand sides of 4000 rows run on the resident engine, which needs two vectors each; what is taken and
+    what refused goes by the nine of the one-workgroup engine, which has to fit as well:
+    (9 nrhs + 1) 4000 doubles of 56 MiB."""
+    from phipict_amd import _lib, profiling
+
+    assert ((9 * nrhs + 1) * 4000 * 8 <= 56 << 20) == fits
+    t, b, x = _grid_case(80, 50, nrhs)
+    before = profiling.resident_counts()
+    rc, res = _call("pp_solve_linear_noalloc", _desc(*t), b, x, nrhs, 1e-8, False, False)
+    after = profiling.resident_counts()
+    assert after[1:] == before[1:] and after[0] - before[0] == int(fits)
+    if fits:
+        assert rc == 0 and all(r[2] for r in res)
+    else:
+        assert rc != 0 and b"scratch maximum" in _lib.LIB.pp_last_error() and float(x.abs().max()) == 0.0
+
+
+def test_noalloc_largest_resident_plan():
+    """524288 rows on 256 workgroups of four rows per thread: the exchanged words fit the static scratch."""
+    from phipict_amd import profiling
+
+    t, b, x = _grid_case(1024, 512, 1)
+    x_ref = torch.zeros_like(x)
+    before = profiling.resident_counts()
+    rc1, res1 = _call("pp_solve_linear", _desc(*t), b, x_ref, 1, 1e-8, False, False)
+    rc2, res2 = _call("pp_solve_linear_noalloc", _desc(*t), b, x, 1, 1e-8, False, False)
+    assert rc1 == 0 and rc2 == 0 and res1 == res2 and torch.equal(x, x_ref)
+    assert tuple(a - b for a, b in zip(profiling.resident_counts(), before)) == (2, 0, 0)
