@@ -178,8 +178,9 @@ __device__ __forceinline__ bool team_decide(Team &tm, const double (&v)[NQ], Tea
 
 // What a workgroup works on.
 struct Share {
-    int piece, n, vbase, mrow, row0; // result index, rows, vector offset, matrix row offset, first own row
-    int m;                           // matrix of a batch
+    int piece, n, mrow, row0; // result index, rows, matrix row offset, first own row
+    size_t vbase;             // vector offset
+    int m;                    // matrix of a batch
     double scale;
 };
 template <typename T>
@@ -202,7 +203,7 @@ __device__ __forceinline__ Share share_of(const ResArgs<T> &a, Team &tm, int row
         tm.G = a.G;
         s.piece = a.team0 + team;
         s.n = a.n;
-        s.vbase = s.piece * a.n;
+        s.vbase = (size_t)s.piece * a.n;
         s.mrow = 0;
         s.m = s.piece / a.rpm;
         s.scale = a.scale;
@@ -315,7 +316,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
         }
     const T *dv = a.dinv ? a.dinv + (size_t)sh.m * a.dinvStride + sh.row0 : nullptr;
     const int own = sh.n - sh.row0; // rows k with t + k * blk < own belong to this thread
-    const size_t v0 = (size_t)sh.vbase + sh.row0 + t; // vector offset of the thread's first row
+    const size_t v0 = sh.vbase + sh.row0 + t; // vector offset of the thread's first row
     T x[R], r[R], p[R];
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -353,7 +354,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     auto gather = [&](int k, unsigned tag, T (&out)[EW], Patience &left) {
         Tagged<T> g[EW];
         int c[EW];
-        const word_t *Z = zpar(tag) + ((size_t)sh.vbase - a.zorigin) * TW;
+        const word_t *Z = zpar(tag) + (sh.vbase - a.zorigin) * TW;
 #pragma unroll
         for (int j = 0; j < EW; ++j) {
             c[j] = hide(M.c[k][j]);
@@ -393,7 +394,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
 #pragma unroll
                 for (int j = 0; j < EW; ++j) {
                     const int c = M.c[k][j] >= 0 ? sh.row0 + M.c[k][j] : -1 - M.c[k][j];
-                    ax += M.a[k][j] * a.x[(size_t)sh.vbase + c];
+                    ax += M.a[k][j] * a.x[sh.vbase + c];
                 }
                 const T bi = rhs(k);
                 r[k] = bi - ax;

@@ -110,6 +110,35 @@ def test_residual_replacement_in_large_teams(shape):
     _check(*_grid_operator(shape), 1, np.float64, residualResetSteps=7)
 
 
+def test_batch_of_more_values_than_32_bits_count():
+    """2^31 + 2^20 values in right-hand sides of 4096 rows, one workgroup each: offsets into the vectors."""
+    import phipict_amd as pa
+
+    row, col, val = _grid_operator((64, 64))
+    val = np.where(val > 0, val + 16.0, val)
+    n, nrhs = 4096, (1 << 19) + 256
+    print(f"[resident] {nrhs} right-hand sides of {n} rows f32", flush=True)
+    A = pa.CSRmatrix(torch.as_tensor(val, dtype=torch.float32, device=DEV), torch.as_tensor(col, device=DEV),
+                     torch.as_tensor(row, device=DEV))
+    b = torch.empty(nrhs * n, dtype=torch.float32, device=DEV)
+    b.normal_(generator=torch.Generator(DEV).manual_seed(3))
+    x = torch.zeros_like(b)
+    try:
+        with resident(finished=1):
+            infos = pa.SolveLinear(A, b, x, maxIterations=100, tolerance=1e-4)
+        assert all(i.converged for i in infos)
+        r = np.repeat(np.arange(n), np.diff(row))
+        for k in (0, (1 << 19) - 1, 1 << 19, nrhs - 1):
+            xk, bk = (v[k * n:(k + 1) * n].cpu().numpy().astype(np.float64) for v in (x, b))
+            res = bk - np.bincount(r, weights=val * xk[col], minlength=n)
+            # the stopping residual, and the rounding of FP32 in sums of ~40 |x|
+            assert np.linalg.norm(res) <= np.sqrt(n) * 1e-4 + 40 * 8 * np.finfo(np.float32).eps * np.linalg.norm(xk), k
+    finally:
+        del b, x
+        pa.ReleaseKrylovWorkspaces()
+        torch.cuda.empty_cache()
+
+
 @contextmanager
 def no_waiting():
     """Teams of several workgroups give up at the first word that is not there yet."""
