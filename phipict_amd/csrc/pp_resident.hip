@@ -22,11 +22,12 @@
 //
 // A team member that waits too long (some other process or a fault keeps a workgroup of the team from
 // running) gives up, and says so in the launch's `failed` word: the host then puts the start guess back,
-// which teams that finished have overwritten, and runs the solve on the multi-launch engine. A thread spends RES_SPINS polls at most on the words of one vector and, in the
-// wave that folds, as many on the sums; polls left after a workgroup has given up anywhere in the launch
-// are not made, and a workgroup whose vector did not arrive does not wait for sums. Teams are as large as the chip, not larger,
-// and one launch of several-workgroup teams runs at a time per process (the host holds a lock), so
-// that all members are resident together.
+// which teams that finished have overwritten, and runs the solve on the multi-launch engine. A thread
+// spends RES_SPINS polls at most on the words of one vector and, in the wave that folds, as many on the
+// sums; polls left after a workgroup has given up anywhere in the launch are not made, and a workgroup
+// whose vector did not arrive does not wait for sums. The launches of several-workgroup teams that a
+// process has on a device have at most one workgroup per CU together (pp_gate.hpp), so that all members
+// are resident together.
 //
 // Recurrences and stopping rules are those of the other engines (pp_krylov.hpp); every thread
 // applies them to its own copy of the record, from sums folded in one fixed order by every workgroup.

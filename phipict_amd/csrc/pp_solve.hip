@@ -18,6 +18,7 @@
 // Recurrences, stopping rules and reported iteration counts restate the reference's fused
 // solvers (csrc/phipict/solvers/krylov/krylov.cu: CG :291-568, BiCGStab :598-824, AMG-PCG
 // :1389-1546 with the V-cycle :1247-1385); the rules themselves are in pp_krylov.hpp.
+#include "pp_gate.hpp"
 #include "pp_resident.hpp"
 
 #include <algorithm>
@@ -1177,6 +1178,7 @@ struct ThreadSpaces {
     int *tbad = nullptr;
     int64_t resident[3] = {0, 0, 0}; // solves the resident engine finished, declined and gave up on
     int residentSpins = RES_SPINS;
+    bool usesTeams = false; // has launched teams of several workgroups
 };
 static std::vector<ThreadSpaces *> g_all_spaces; // every thread's, for pp_release_workspaces
 
@@ -1210,6 +1212,9 @@ static int cu_count() {
     }
     return cus;
 }
+
+// Workgroups of team launches that run at once.
+static int resident_cus() { return std::min(cu_count(), RES_WG); }
 
 // Workgroups per grid row of a phase kernel: enough for every row, at most PHASE_THREADS per CU shared by
 // the grid rows (the partial sets are folded by every workgroup of the next launch, so the
@@ -1657,8 +1662,39 @@ static int bicg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const
 }
 
 // ---------------- the resident engine ----------------
-// Launches with teams of several workgroups run one at a time: every member must be resident.
-static std::mutex g_resident_lock;
+// A launch of teams of several workgroups, from before it is queued until its kernels have ended: the
+// members have to run at once, so the launches of all threads together have at most a workgroup per CU
+// of their device (other kernels end by themselves). Where several threads solve, the share is taken only once the
+// stream's earlier work is done, so that none waits for what another has queued before its solve.
+constexpr int TEAM_DEVICES = 64;
+static TeamGate g_team_gates[TEAM_DEVICES];
+static std::atomic<int> g_team_threads{0};
+
+class TeamShare {
+public:
+    ~TeamShare() {
+        if (gate) gate->leave(need);
+    }
+    int take(int workgroups, hipStream_t s) {
+        int dev = 0;
+        PP_HIP(hipGetDevice(&dev));
+        ThreadSpaces &ts = my_spaces();
+        if (!ts.usesTeams) {
+            ts.usesTeams = true;
+            ++g_team_threads;
+        }
+        if (g_team_threads > 1) PP_HIP(hipStreamSynchronize(s));
+        TeamGate &g = g_team_gates[dev % TEAM_DEVICES];
+        need = workgroups;
+        g.enter(need, resident_cus());
+        gate = &g;
+        return PP_OK;
+    }
+
+private:
+    TeamGate *gate = nullptr;
+    int need = 0;
+};
 
 // How a resident solve of `teams` systems of n rows runs: one workgroup each, or teams of G
 // workgroups with R rows per thread, `perLaunch` teams at a time. ew 0: not on this engine.
@@ -1695,7 +1731,7 @@ static ResPlan resident_plan(int n, int teams, int ew) {
         p.ew = ew;
         return p;
     }
-    const int cus = std::min(cu_count(), RES_WG);
+    const int cus = resident_cus();
     for (int R : {1, 2, 4}) {
         const int G = (n + RES_WG * R - 1) / (RES_WG * R);
         const int fit = cus / G;
@@ -1797,9 +1833,9 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
     const int launches = (B + plan.perLaunch - 1) / plan.perLaunch;
     if (!plan.local && (uint64_t)tags * launches > (1u << 31)) return PP_OK;
     if (sp.fixed && (zWords + slotWords) * sizeof(uint64_t) > sp.linkCap) return PP_OK;
-    std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
-    if (!plan.local) alone.lock();
+    TeamShare share;
     if (!plan.local) {
+        if (int e = share.take(maxWgs, s)) return e;
         uint32_t tag = 0;
         if (int e = resident_link(sp, zWords + slotWords, tags * (uint32_t)launches, s, &tag)) return e;
         a.zbuf = reinterpret_cast<unsigned long long *>(sp.link);
@@ -2643,7 +2679,7 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
         len[k] = segRows[p + 1] - segRows[p];
         mrow[k] = segRows[p];
     }
-    const SegPack pack = seg_pack(len, ew, std::min(cu_count(), RES_WG));
+    const SegPack pack = seg_pack(len, ew, resident_cus());
     if (!pack.R) return PP_OK;
     const uint32_t tags = resident_tags(maxit);
     if ((uint64_t)tags * std::max(1, pack.launches) > (1u << 31)) return PP_OK;
@@ -2665,9 +2701,11 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
     a.ntols = ntols > RES_TOLS ? 1 : ntols;
     for (int k = 0; k < a.ntols; ++k) a.tols[k] = tols[k];
     a.tolsDev = ntols > RES_TOLS ? (const double *)sp.tols : nullptr;
-    std::unique_lock<std::mutex> alone(g_resident_lock, std::defer_lock);
+    TeamShare share;
     if (pack.launches) {
-        alone.lock();
+        int most = 0;
+        for (int l = 0; l < pack.launches; ++l) most = std::max(most, pack.wgFirst[l + 1] - pack.wgFirst[l]);
+        if (int e = share.take(most, s)) return e;
         const size_t zWords = 2 * a.vecLen * (sizeof(T) / 4);
         uint32_t tag = 0;
         if (int e = resident_link(sp, zWords + (size_t)2 * 3 * RES_WG * 2, tags * (uint32_t)pack.launches, s, &tag)) return e;

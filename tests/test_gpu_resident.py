@@ -139,6 +139,75 @@ def test_batch_of_more_values_than_32_bits_count():
         torch.cuda.empty_cache()
 
 
+def test_threads_do_not_wait_for_each_others_queued_work():
+    """A thread with a second of products queued on its stream before its solve, and a thread that solves
+    meanwhile on another: the second is done long before the first one's queue is. Then both solve at once,
+    over and over, in teams that fit the device together and teams that do not."""
+    import threading
+
+    import phipict_amd as pa
+    from phipict_amd import profiling
+
+    def system(shape):
+        row, col, val = _grid_operator(shape)
+        n = row.size - 1
+        A = pa.CSRmatrix(*(torch.as_tensor(a, device=DEV) for a in (val, col, row)))
+        b = torch.as_tensor(np.random.default_rng(n).standard_normal(n), device=DEV)
+        x = torch.zeros(n, dtype=torch.float64, device=DEV)
+        ref = torch.zeros_like(x)
+        pa.SolveLinear(A, b, ref, maxIterations=4000, tolerance=1e-9)
+        return A, b, x, ref
+
+    def solve(s):
+        A, b, x, ref = s
+        x.zero_()
+        info = pa.SolveLinear(A, b, x, maxIterations=4000, tolerance=1e-9)[0]
+        assert info.converged and torch.equal(x, ref)
+
+    small = [system((70, 65)), system((90, 70))]
+    large = [system((400, 200)), system((300, 290))]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    m = torch.randn(2048, 2048, device=DEV)
+    out = torch.empty_like(m)
+    queued, end = threading.Event(), torch.cuda.Event()
+    seen, counts, errors = {}, [None, None], []
+    line = threading.Barrier(2, timeout=60)
+
+    def run(me):
+        try:
+            before = profiling.resident_counts()
+            with torch.cuda.stream(streams[me]):
+                solve(small[me])  # both threads have their workspaces
+                line.wait()
+                if me == 0:
+                    for _ in range(6000):
+                        torch.mm(m, m, out=out)
+                    end.record()
+                    queued.set()
+                    solve(small[0])
+                else:
+                    queued.wait(60)
+                    solve(small[1])
+                    seen["busy"] = not end.query()
+                line.wait()
+                for s in (small[me], large[me]) * 20:
+                    solve(s)
+            counts[me] = tuple(b - a for a, b in zip(before, profiling.resident_counts()))
+        except BaseException as e:  # reported below, in the test's own thread
+            errors.append(e)
+            line.abort()
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(100)
+    assert not errors, errors
+    assert seen["busy"]
+    assert counts == [(42, 0, 0)] * 2
+
+
 @contextmanager
 def no_waiting():
     """Teams of several workgroups give up at the first word that is not there yet."""
