@@ -2960,6 +2960,7 @@ int pp_solve_linear_noalloc(const pp_csr *A, const void *rhs, void *x, int32_t n
                             const double *tols, int32_t ntols, int32_t criterion, int32_t use_bicg,
                             int32_t matrix_rank_deficient, int32_t residual_reset_steps, int32_t transpose_a,
                             int32_t return_best, void *stream, pp_solve_result *results) {
+    (void)my_spaces(); // a thread's first use takes g_lock
     std::lock_guard<std::mutex> lock(g_lock);
     Space *sp = nullptr;
     if (int e = fixed_space(&sp)) return e;

@@ -135,3 +135,16 @@ def test_noalloc_largest_resident_plan():
     rc2, res2 = _call("pp_solve_linear_noalloc", _desc(*t), b, x, 1, 1e-8, False, False)
     assert rc1 == 0 and rc2 == 0 and res1 == res2 and torch.equal(x, x_ref)
     assert tuple(a - b for a, b in zip(profiling.resident_counts(), before)) == (2, 0, 0)
+
+
+def test_a_threads_first_solve_may_be_allocation_free():
+    import threading
+
+    t, b, x = _grid_case(40, 30, 1)
+    torch.cuda.synchronize()
+    got = []
+    th = threading.Thread(target=lambda: got.append(_call("pp_solve_linear_noalloc", _desc(*t), b, x, 1, 1e-8, False, False)),
+                          daemon=True)
+    th.start()
+    th.join(30)
+    assert got and got[0][0] == 0 and got[0][1][0][2]
