@@ -17,7 +17,7 @@ from typing import Any, Callable, Optional
 import numpy as np
 import torch
 
-from . import ops
+from . import ops, profiling
 from .domain import CSRmatrix, Domain, transform_size
 from .hooks import Hook, Hooks
 from .solvers import amg as amg_mod
@@ -95,12 +95,17 @@ def tune_segment_tiles(A: CSRmatrix, segments, rhs: torch.Tensor, use_BiCG: bool
     side component for each
     candidate tile size with HIP events on the current stream and keeps the fastest. Larger
     tiles mean fewer workgroups and shorter folds, smaller ones more parallelism on small
-    instances."""
+    instances. CG that runs on the resident engine has no tiles; BiCGStab, whose solves of the same
+    instances will use the choice, is timed in its place."""
     n = A.getRows()
     b = rhs.reshape(-1)[:n].contiguous()
     if not b.is_cuda:
         return 1024
     x = torch.zeros_like(b)
+    if not use_BiCG:
+        before = profiling.resident_counts()[0]
+        ops.SolveSegmented(A, segments, b, x, maxIterations=2, tolerance=0.0)
+        use_BiCG = profiling.resident_counts()[0] > before
     timings = {}
     for tile in SEGMENT_TILE_CANDIDATES:
         if tile > max(256, n):

@@ -227,6 +227,27 @@ def test_64_uneven_instances_step_like_solo_runs():
     print(f"  worst rel L2 over 64 instances: {worst:.2e}", flush=True)
 
 
+def test_tile_tuner_times_the_engine_that_has_tiles():
+    """A tile size tuned on a CG solve of the resident engine, which has no tiles, is timed on BiCGStab."""
+    import phipict_amd as pa
+    from phipict_amd import profiling
+
+    parts = _operators(False)
+    row, col, val = _block_diag(parts)
+    segs = np.concatenate([[0], np.cumsum([p[0].size - 1 for p in parts])])
+    A = pa.CSRmatrix(torch.as_tensor(val, device=DEV), torch.as_tensor(col, device=DEV), torch.as_tensor(row, device=DEV))
+    b = torch.as_tensor(np.random.default_rng(9).standard_normal(row.size - 1), device=DEV)
+    profiling.start(1)
+    try:
+        tile = pa.simulation.tune_segment_tiles(A, segs, b)
+    finally:
+        profiling.stop()
+    launched = {t.name: t.launches for t in profiling.read()}
+    assert tile in pa.simulation.SEGMENT_TILE_CANDIDATES
+    tried = pa.simulation.SEGMENT_TUNING_LOG[-1][2]
+    assert launched.get("seg_bicg", 0) >= 24 * len(tried) and launched.get("cg_small", 0) == 1, launched
+
+
 def test_captured_chunks_equal_direct_launches():
     """useGraphs: the segmented solves replayed from captured HIP graphs give bit-identical
     solutions and results to direct launches, over repeated calls (replays of cached graphs)."""
