@@ -41,6 +41,16 @@ struct SolveRec {
     int32_t zero; // the right-hand side is exactly zero
 };
 
+// A record to or from memory, field by field. Copied as a block, the fields that a kernel does not name stay a
+// local array, which the compiler puts into LDS or scratch; to find its place in LDS every wave then
+// reads the dispatch packet, which lies in host memory: 7-10 us at the start of a kernel of 8-20.
+__host__ __device__ __forceinline__ void rec_copy(SolveRec &d, const SolveRec &s) {
+    d.tol = s.tol; d.rho = s.rho; d.alpha = s.alpha; d.omega = s.omega;
+    d.crit = s.crit; d.best = s.best; d.prev = s.prev; d.half = s.half;
+    d.iter = s.iter; d.maxit = s.maxit; d.report = s.report; d.bestAt = s.bestAt;
+    d.climb = s.climb; d.fate = s.fate; d.flags = s.flags; d.zero = s.zero;
+}
+
 template <typename T>
 struct Csr {
     const int32_t *__restrict__ row;

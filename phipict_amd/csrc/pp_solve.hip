@@ -176,10 +176,11 @@ __device__ __forceinline__ void decide_each(Head<NB, T> &H, const SolveRec *in, 
     for (int k = 0; k < NB; ++k) {
         int act = 0;
         if (k < sp.count) {
-            SolveRec R = in[sp.first + k];
+            SolveRec R;
+            rec_copy(R, in[sp.first + k]);
             decide(k, R);
             act = rec_active(R);
-            if (out && blockIdx.x == 0 && lead) out[sp.first + k] = R;
+            if (out && blockIdx.x == 0 && lead) rec_copy(out[sp.first + k], R);
         }
         if (lead) H.act[k] = act;
         any |= act;
@@ -2355,7 +2356,8 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, const T *__restrict__ 
                                                 SegParts pqOut, const SolveRec *in, SolveRec *out, int open) {
     __shared__ double lds[16 * 3];
     const Tile t = tile_of(P);
-    SolveRec R = in[t.k];
+    SolveRec R;
+    rec_copy(R, in[t.k]);
     bool act = rec_active(R);
     double tot[2];
     fold<2>(rrIn, 0, t.t0, t.t1, tot, lds);
@@ -2371,7 +2373,7 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, const T *__restrict__ 
         }
         act = rec_active(R);
     }
-    if (t.lead && threadIdx.x == 0) out[t.k] = R;
+    if (t.lead && threadIdx.x == 0) rec_copy(out[t.k], R);
     double acc[1] = {0.0};
     if (act) {
         const bool fresh = R.flags & R_FRESH;
@@ -2399,7 +2401,8 @@ __global__ void __launch_bounds__(WG) k_cg_step(T *__restrict__ r, const T *__re
                                                 const SolveRec *in, SolveRec *out) {
     __shared__ double lds[16 * 3];
     const Tile t = tile_of(P);
-    SolveRec R = in[t.k];
+    SolveRec R;
+    rec_copy(R, in[t.k]);
     bool act = rec_active(R);
     double pq[1];
     fold<1>(pqIn, 0, t.t0, t.t1, pq, lds);
@@ -2409,7 +2412,7 @@ __global__ void __launch_bounds__(WG) k_cg_step(T *__restrict__ r, const T *__re
         R.flags &= ~R_FRESH;
         act = rec_active(R);
     }
-    if (t.lead && threadIdx.x == 0) out[t.k] = R;
+    if (t.lead && threadIdx.x == 0) rec_copy(out[t.k], R);
     double acc[3] = {0.0, 0.0, 0.0};
     if (act)
         PP_TILE_ROWS(i, t) {
@@ -2430,7 +2433,8 @@ __global__ void __launch_bounds__(WG) k_bi_dir(const T *__restrict__ r, T *__res
                                                Pieces P, SegParts rrIn, const SolveRec *in, SolveRec *out, int open) {
     __shared__ double lds[16 * 2];
     const Tile t = tile_of(P);
-    SolveRec R = in[t.k];
+    SolveRec R;
+    rec_copy(R, in[t.k]);
     bool act = rec_active(R);
     double tot[2];
     fold<2>(rrIn, 0, t.t0, t.t1, tot, lds);
@@ -2445,7 +2449,7 @@ __global__ void __launch_bounds__(WG) k_bi_dir(const T *__restrict__ r, T *__res
         }
         act = rec_active(R);
     }
-    if (t.lead && threadIdx.x == 0) out[t.k] = R;
+    if (t.lead && threadIdx.x == 0) rec_copy(out[t.k], R);
     if (!act) return;
     const bool fresh = R.flags & R_FRESH;
     const T omega = T(R.omega);
@@ -2481,7 +2485,8 @@ __global__ void __launch_bounds__(WG) k_bi_stab(Csr<T> A, const T *__restrict__ 
                                                 const SolveRec *in) {
     __shared__ double lds[16 * 3];
     const Tile t = tile_of(P);
-    SolveRec R = in[t.k];
+    SolveRec R;
+    rec_copy(R, in[t.k]);
     double r0v[1];
     fold<1>(r0vIn, 0, t.t0, t.t1, r0v, lds);
     T alpha = T(0);
@@ -2517,7 +2522,8 @@ __global__ void __launch_bounds__(WG) k_bi_step(T *__restrict__ r, const T *__re
                                                 const SolveRec *in, SolveRec *out) {
     __shared__ double lds[16 * 3];
     const Tile t = tile_of(P);
-    SolveRec R = in[t.k];
+    SolveRec R;
+    rec_copy(R, in[t.k]);
     bool act = rec_active(R);
     double r0v[1], ts[3];
     fold<1>(r0vIn, 0, t.t0, t.t1, r0v, lds);
@@ -2531,7 +2537,7 @@ __global__ void __launch_bounds__(WG) k_bi_step(T *__restrict__ r, const T *__re
         if (half) rule_bicg_half_met(R);
         R.flags &= ~R_FRESH;
     }
-    if (t.lead && threadIdx.x == 0) out[t.k] = R;
+    if (t.lead && threadIdx.x == 0) rec_copy(out[t.k], R);
     double acc[2] = {0.0, 0.0};
     if (act) {
         const T alpha = T(R.alpha), omega = T(R.omega);
