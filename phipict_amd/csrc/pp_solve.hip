@@ -76,11 +76,12 @@ __device__ __forceinline__ void put_parts(const Parts &P, double (&acc)[NB][NQ],
 
 // Totals of quantities q0..q0+NQ-1 of right-hand sides first..first+count-1, folded over the G
 // partials in a fixed order by one wavefront and left in out[k * NQ + q] (LDS): every workgroup
-// of a launch obtains the same bits. The loads of FOLD_AHEAD strides and of all quantities are in
-// flight together.
-constexpr int FOLD_AHEAD = 8;
+// of a launch obtains the same bits. The loads of fold_ahead(NB * NQ) strides and of all quantities are
+// in flight together.
+constexpr int fold_ahead(int sums) { return sums <= 3 ? 8 : (sums >= 12 ? 2 : 24 / sums); }
 template <int NB, int NQ>
 __device__ __forceinline__ void fold(const Parts &P, int q0, int first, int count, double *out) {
+    constexpr int FOLD_AHEAD = fold_ahead(NB * NQ);
     const int lane = threadIdx.x & 63;
     double acc[NB * NQ];
 #pragma unroll
@@ -167,25 +168,28 @@ __device__ __forceinline__ void row_each(const Csr<T> &A, const T *__restrict__ 
 #define PP_ROWS(i, n) for (int i = blockIdx.x * NT + (int)threadIdx.x; i < (n); i += gridDim.x * NT)
 
 // Runs decide(k, R) for every right-hand side of the span in the first wavefront, on a copy of its
-// record: k's step, flag and whether it stays active go to H, the record to `out` (workgroup 0).
+// record: k's step, flag and whether it stays active go to H, the record to `out` (workgroup 0). Several
+// right-hand sides are decided at once, each by a lane of its own: one after another, with a cold load
+// and several divisions each, they cost about a microsecond per right-hand side and kernel. Lanes that may
+// write to H: decider().
+template <int NB>
+__device__ __forceinline__ bool decider() { return NB > 1 || threadIdx.x == 0; }
 template <int NB, typename T, typename F>
 __device__ __forceinline__ void decide_each(Head<NB, T> &H, const SolveRec *in, SolveRec *out, const Span &sp, F decide) {
-    const bool lead = threadIdx.x == 0;
-    int any = 0;
-#pragma unroll 1
-    for (int k = 0; k < NB; ++k) {
-        int act = 0;
-        if (k < sp.count) {
-            SolveRec R;
-            rec_copy(R, in[sp.first + k]);
-            decide(k, R);
-            act = rec_active(R);
-            if (out && blockIdx.x == 0 && lead) rec_copy(out[sp.first + k], R);
-        }
-        if (lead) H.act[k] = act;
-        any |= act;
+    const int lane = threadIdx.x;
+    const int k = NB > 1 ? lane : 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the totals in H, written by lane 0
+    int act = 0;
+    if (k < sp.count) {
+        SolveRec R;
+        rec_copy(R, in[sp.first + k]);
+        decide(k, R);
+        act = rec_active(R);
+        if (out && blockIdx.x == 0 && decider<NB>()) rec_copy(out[sp.first + k], R);
     }
-    if (lead) H.any = any;
+    if (k < NB && decider<NB>()) H.act[k] = act;
+    const int any = NB > 1 ? __any(act) : act;
+    if (lane == 0) H.any = any;
 }
 
 // Control of a phase kernel, passed by value.
@@ -311,7 +315,7 @@ __global__ void __launch_bounds__(WG) k_cg_turn(Csr<T> A, T *__restrict__ r, con
                 }
                 if (mode == TURN_STEP_RESET && rec_active(R)) R.flags |= R_FRESH | R_RESET;
             }
-            if (threadIdx.x == 0) {
+            if (decider<NB>()) {
                 H.step[k] = beta;
                 H.flag[k] = R.flags & R_FRESH;
             }
@@ -409,7 +413,7 @@ __global__ void __launch_bounds__(NT) k_cg_step(int n, int rpm, T *__restrict__ 
                 alpha = T(rule_alpha(R, H.tot[k]));
                 R.flags &= ~(R_FRESH | R_RESET);
             }
-            if (threadIdx.x == 0) {
+            if (decider<NB>()) {
                 H.step[k] = alpha;
                 H.flag[k] = xbest && (R.flags & R_KEEP);
             }
@@ -542,7 +546,7 @@ __global__ void __launch_bounds__(WG) k_bicg_stab(Csr<T> A, const T *__restrict_
         fold<NB, 1>(r0vIn, 0, sp.first, sp.count, H.tot);
         decide_each<NB>(H, ph.in, nullptr, sp, [&](int k, SolveRec &R) {
             const T alpha = rec_active(R) ? T(rule_alpha(R, H.tot[k])) : T(0);
-            if (threadIdx.x == 0) H.step[k] = alpha;
+            if (decider<NB>()) H.step[k] = alpha;
         });
     }
     __syncthreads();
@@ -1536,8 +1540,23 @@ static void cg_large_grid(int n, int B, int rpm, int *rows, int *G) {
     *G = phase_width(n, *rows, WG);
 }
 
+// Dynamic LDS of a row pass over plain CSR for several right-hand sides, which it does not use: it bounds the
+// workgroups per CU. Each work-item walks a row of its own, so a line of the matrix is wanted again for
+// every next entry, and more rows in flight than CSR_FLIGHT bytes of entries push each other out of
+// the caches. 1 M rows of nine entries, three right-hand sides, 20 iterations: 3.6 ms with two
+// workgroups per CU (FP64), 4.6 with four, 5.1 with eight; in FP32 3.0, 2.3 and 3.3; 1 M rows of seven
+// entries 3.3, 3.1, 3.8 and 2.9, 2.0, 2.4; 630 k rows of five entries 2.2, 1.7, 2.0 and 2.0, 1.5, 1.4.
+constexpr size_t CSR_FLIGHT = 80 << 10, CU_LDS = 160 << 10;
 template <typename T>
-static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const double *tols, int ntols, double scale,
+static size_t csr_flight_lds(const Csr<T> &A, long nnz, int NB) {
+    if (A.ell_w > 0 || NB < 2) return 0;
+    const size_t rows = size_t(WG) * nnz / A.n * (sizeof(T) + sizeof(int32_t)); // of one workgroup
+    const size_t wgs = std::max<size_t>(2, CSR_FLIGHT / std::max<size_t>(1, rows));
+    return wgs >= PHASE_THREADS / WG ? 0 : CU_LDS / (wgs + 1) + 1024;
+}
+
+template <typename T>
+static int cg_large(const Csr<T> &A, long nnz, const T *b, T *x, int B, int maxit, const double *tols, int ntols, double scale,
                     int resetEvery, int returnBest, int project, int jacobi, Space &sp, hipStream_t s,
                     pp_solve_result *res) {
     const int n = A.n;
@@ -1560,6 +1579,7 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
     const Parts sSum = pc.take(B, 1, G), sRR = pc.take(B, 3, G), sPQ = pc.take(B, 1, G), sRst = pc.take(B, 2, G);
     SolveRec *ra = recs_a(sp), *rb = recs_b(sp, B);
     const dim3 grid(G, rows), block(WG);
+    const size_t turnLds = csr_flight_lds(A, nnz, NBv);
     hipLaunchKernelGGL(k_init_recs, dim3(1), dim3(64), 0, s, ra, B, tols[0], ntols > 1 ? (const double *)sp.tols : nullptr, maxit);
     if (jacobi) launch_jacobi<T>(A, numMat, V(V_COUNT), s);
     if (project) hipLaunchKernelGGL((k_sum<T, WG>), dim3(G, B), block, 0, s, b, n, sSum);
@@ -1567,27 +1587,27 @@ static int cg_large(const Csr<T> &A, const T *b, T *x, int B, int maxit, const d
     PP_JAC_CASE(jacobi, PP_NB_CASE(NBv, PP_EW_CASE(A.ell_w,
         hipLaunchKernelGGL((k_open<T, NB, EW, JAC, WG>), grid, block, 0, s, A, b, project ? sSum : Parts{nullptr, 1, G},
                            project ? bw : (T *)nullptr, x, r, (T *)nullptr, B, sRR, jac);
-        hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, 0, s, A, r, p[0], p[1], q, x, bw, sRR, sPQ, sRst,
+        hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, turnLds, s, A, r, p[0], p[1], q, x, bw, sRR, sPQ, sRst,
                            openPh, (int)TURN_OPEN, jac))));
     PP_LAUNCH_CHECK();
     const Phase stepPh{rb, ra, B, scale, returnBest}, turnPh{ra, rb, B, scale, returnBest};
     const Phase afterPh{rb, nullptr, B, scale, returnBest};
     auto body = [&](hipStream_t st, int j) {
         const int cur = 1 ^ (j & 1); // the opening turn wrote p[1]
-        const bool reset = resetEvery > 0 && (j + 1) % resetEvery == 0;
+        const bool reset = resetEvery > 0 && (j + 1) % resetEvery == 0, wasReset = resetEvery > 0 && j > 0 && j % resetEvery == 0;
         PP_JAC_CASE(jacobi, PP_NB_CASE(NBv,
             PP_TIMED(PP_K_CG_UPDATE, n, st,
                 hipLaunchKernelGGL((k_cg_step<T, NB, JAC, WG>), grid, block, 0, st, n, A.rpm, r, p[cur], q, x, xbest, sPQ,
-                                   sRst, sRR, stepPh, jac));
+                                   wasReset ? sRst : Parts{nullptr, 2, G}, sRR, stepPh, jac));
             PP_EW_CASE(A.ell_w,
                 if (reset) {
-                    hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, 0, st, A, r, p[cur], p[cur ^ 1], q, x, bw,
+                    hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, turnLds, st, A, r, p[cur], p[cur ^ 1], q, x, bw,
                                        sRR, sPQ, sRst, turnPh, (int)TURN_STEP_RESET, jac);
-                    hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, 0, st, A, r, p[cur], p[cur ^ 1], q, x, bw,
+                    hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, turnLds, st, A, r, p[cur], p[cur ^ 1], q, x, bw,
                                        sRR, sPQ, sRst, afterPh, (int)TURN_AFTER_RESET, jac);
                 } else {
                     PP_TIMED(PP_K_CG_DIRECTION, n, st,
-                        hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, 0, st, A, r, p[cur], p[cur ^ 1], q, x,
+                        hipLaunchKernelGGL((k_cg_turn<T, NB, EW, JAC>), grid, block, turnLds, st, A, r, p[cur], p[cur ^ 1], q, x,
                                            bw, sRR, sPQ, sRst, turnPh, (int)TURN_STEP, jac));
                 })));
     };
@@ -2902,7 +2922,7 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
             return small_solve<T>(C, b, xx, nrhs, maxit, tols, ntols, scale, use_bicg ? 0 : residual_reset_steps,
                                   return_best, matrix_rank_deficient, use_bicg, jacobi, sp, s, results);
         if (use_bicg) return bicg_large<T>(C, b, xx, nrhs, maxit, tols, ntols, scale, jacobi, sp, s, results);
-        return cg_large<T>(C, b, xx, nrhs, maxit, tols, ntols, scale, residual_reset_steps, return_best,
+        return cg_large<T>(C, A->nnz, b, xx, nrhs, maxit, tols, ntols, scale, residual_reset_steps, return_best,
                            matrix_rank_deficient, jacobi, sp, s, results);
     });
     return PP_OK;
