@@ -300,6 +300,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     if (*a.declined == a.done) return;
     Team tm;
     const Share sh = share_of(a, tm, blk * R);
+    if (a.onlyHeld && a.recs[sh.piece].zero != ZERO_HELD) return;
     tm.slots = a.slots;
     tm.tag = a.tag;
     tm.fresh = Patience{a.spins, a.failed, a.done};
@@ -414,6 +415,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
                     S.fate = F_MET;
                     S.report = 0;
                     S.crit = 0.0;
+                    S.zero = a.zeroStops;
                 }
                 o.active = rec_active(S);
                 o.fresh = 1;
@@ -535,7 +537,7 @@ __global__ void __launch_bounds__(LOCAL ? RES_LOCAL_WG : RES_WG) k_resident_cg(R
     }
     const SolveRec &S = L.S;
     const bool best = a.xbest && (S.fate == F_EXHAUSTED || S.fate == F_STALLED) && S.bestAt >= 0 && S.best < S.crit;
-    const bool zero = S.zero && a.zeroStops;
+    const bool zero = S.zero && a.zeroStops == ZERO_SOLVED;
 #pragma unroll
     for (int k = 0; k < R; ++k)
         if (t + k * blk < own) a.x[v0 + k * blk] = zero ? T(0) : (best ? a.xbest[v0 + k * blk] : x[k]);

@@ -13,6 +13,10 @@ constexpr int RES_LOCAL_WG = 1024; // threads at most of a one-workgroup team
 constexpr int RES_TOLS = 8;        // tolerances passed by value
 constexpr int RES_SPINS = 1 << 21; // polls a thread spends on one exchange before it gives up, about a microsecond each
 
+// Several right-hand sides are set to x = 0 if all of them are zero, and solved as any other if one is not: a
+// zero one is held (SolveRec::zero = ZERO_HELD) until all are known.
+enum { ZERO_RUNS = 0, ZERO_SOLVED = 1, ZERO_HELD = 2 };
+
 // Pieces of a segmented solve: piece k has len[k] rows at vector offset base[k], its matrix rows
 // start at mrow[k]; workgroup w of the launch works on piece wgPiece[w], whose workgroups are
 // wg0[k] .. wg0[k] + G[k] - 1. All null for a plain solve.
@@ -40,7 +44,8 @@ struct ResArgs {
     int n, rpm, G, team0;        // plain solve: rows, right-hand sides per matrix, workgroups per team, first team
     int wgs;                     // workgroups of the launch
     int maxit, returnBest, project, resetEvery;
-    int zeroStops;               // a zero right-hand side ends at once (x = 0)
+    int zeroStops;               // a zero right-hand side ends at once: ZERO_SOLVED (x = 0) or ZERO_HELD (x kept)
+    int onlyHeld;                // run the right-hand sides held by the launch before, as any other
     double scale;                // 1 / sqrt(n) or 1 (a plain solve)
     double tols[RES_TOLS];       // per right-hand side when tolsDev is null (one: tols[0])
     int ntols;

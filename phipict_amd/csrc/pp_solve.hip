@@ -1808,7 +1808,8 @@ static int resident_status(Space &sp, int B, int ew, bool check, hipStream_t s, 
 // calling thread). Otherwise the `len` values of x are the start guess again: teams that finished
 // beside one that gave up have written theirs, and the engine that takes over is not to start from those.
 template <typename T>
-static int resident_results(Space &sp, int B, size_t len, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran) {
+static int resident_results(Space &sp, int B, size_t len, const ResArgs<T> &a, hipStream_t s, const SolveRec **recs, bool *ran,
+                            bool count = true) {
     PP_HIP(hipMemcpyAsync(sp.snap, a.recs, sizeof(SolveRec) * B + sizeof(unsigned) * (B + 2), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     *recs = reinterpret_cast<const SolveRec *>(sp.snap);
@@ -1816,7 +1817,7 @@ static int resident_results(Space &sp, int B, size_t len, const ResArgs<T> &a, h
     const bool declined = st[B + 1] == a.done;
     *ran = st[B] != a.done && !declined;
     for (int k = 0; k < B; ++k) *ran = *ran && st[k] == a.done;
-    ++my_spaces().resident[*ran ? 0 : (declined ? 1 : 2)];
+    if (count || !*ran) ++my_spaces().resident[*ran ? 0 : (declined ? 1 : 2)];
     if (!*ran && !declined) {
         PP_HIP(hipMemcpyAsync(a.x, a.x0, sizeof(T) * len, hipMemcpyDeviceToDevice, s));
         PP_HIP(hipStreamSynchronize(s)); // x0 lies in a workspace that the next engine may grow
@@ -1852,13 +1853,14 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
     const size_t zWords = plan.local ? 0 : 2 * a.vecLen * (sizeof(T) / 4), slotWords = plan.local ? 0 : (size_t)2 * 3 * maxWgs * 2;
     const uint32_t tags = resident_tags(maxit);
     const int launches = (B + plan.perLaunch - 1) / plan.perLaunch;
-    if (!plan.local && (uint64_t)tags * launches > (1u << 31)) return PP_OK;
+    const int rounds = launches + (zeroStops == ZERO_HELD ? 1 : 0);
+    if (!plan.local && (uint64_t)tags * rounds > (1u << 31)) return PP_OK;
     if (sp.fixed && (zWords + slotWords) * sizeof(uint64_t) > sp.linkCap) return PP_OK;
     TeamShare share;
     if (!plan.local) {
         if (int e = share.take(maxWgs, s)) return e;
         uint32_t tag = 0;
-        if (int e = resident_link(sp, zWords + slotWords, tags * (uint32_t)launches, s, &tag)) return e;
+        if (int e = resident_link(sp, zWords + slotWords, tags * (uint32_t)rounds, s, &tag)) return e;
         a.zbuf = reinterpret_cast<unsigned long long *>(sp.link);
         a.slots = a.zbuf + zWords;
         a.tag = tag;
@@ -1876,7 +1878,18 @@ static int resident_solve(const Csr<T> &A, const ResPlan &plan, const T *b, T *x
         a.tag += tags;
         sp.linkTag += plan.local ? 0 : tags;
     }
-    return resident_results(sp, B, len, a, s, recs, ran);
+    if (int e = resident_results(sp, B, len, a, s, recs, ran)) return e;
+    if (zeroStops != ZERO_HELD || !*ran || all_zero_rhs(*recs, B)) return PP_OK;
+    bool held = false;
+    for (int k = 0; k < B; ++k) held = held || (*recs)[k].zero == ZERO_HELD;
+    if (!held) return PP_OK;
+    a.onlyHeld = 1;
+    a.zeroStops = ZERO_RUNS;
+    int e = PP_OK;
+    PP_TIMED(PP_K_CG_SMALL, n, s, e = launch_resident_cg<T>(a, plan.ew, plan.R, plan.threads, plan.local, s));
+    if (e) return e;
+    sp.linkTag += plan.local ? 0 : tags;
+    return resident_results(sp, B, len, a, s, recs, ran, false);
 }
 
 // ---------------- small systems ----------------
@@ -2723,7 +2736,7 @@ static int resident_segmented(const Csr<T> &A, long nnz, const int32_t *segRows,
     a.A = A;
     a.b = b; a.x = x; a.x0 = reinterpret_cast<T *>(sp.vec);
     a.vecLen = total;
-    a.maxit = maxit; a.project = project; a.zeroStops = 1;
+    a.maxit = maxit; a.project = project; a.zeroStops = ZERO_SOLVED;
     a.ntols = ntols > RES_TOLS ? 1 : ntols;
     for (int k = 0; k < a.ntols; ++k) a.tols[k] = tols[k];
     a.tolsDev = ntols > RES_TOLS ? (const double *)sp.tols : nullptr;
@@ -2902,7 +2915,7 @@ static int solve_linear(const pp_csr *A, const void *rhs, void *x, int32_t nrhs,
             }
             if (int e = resident_solve<T>(C, plan, b, xx, nrhs, maxit, tols, ntols, scale,
                                           use_bicg ? 0 : residual_reset_steps, return_best, matrix_rank_deficient, use_bicg,
-                                          jacobi, !small && nrhs == 1, sp, s, &recs, &ran))
+                                          jacobi, small ? ZERO_RUNS : (nrhs == 1 ? ZERO_SOLVED : ZERO_HELD), sp, s, &recs, &ran))
                 return e;
             if (ran) {
                 if (!small && all_zero_rhs(recs, nrhs)) {

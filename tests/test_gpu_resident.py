@@ -208,6 +208,38 @@ def test_threads_do_not_wait_for_each_others_queued_work():
     assert counts == [(42, 0, 0)] * 2
 
 
+def test_zero_right_hand_sides_of_a_batch():
+    """All zero: x = 0 without iterating, from any start guess. Some zero: solved as any other, from the start
+    guess, with the oracle's iterations."""
+    import phipict_amd as pa
+    from phipict_amd import profiling
+
+    row, col, val = _grid_operator((200, 200))
+    n, nrhs, tol = 40000, 3, 1e-9
+    A = pa.CSRmatrix(*(torch.as_tensor(a, device=DEV) for a in (val, col, row)))
+    x0 = 1.0 + 0.1 * np.random.default_rng(3).standard_normal(nrhs * n)
+    x = torch.as_tensor(x0.copy(), device=DEV)
+    profiling.start(1)
+    try:
+        with resident(finished=1):
+            infos = pa.SolveLinear(A, torch.zeros_like(x), x, maxIterations=4000, tolerance=tol)
+    finally:
+        profiling.stop()
+    assert all(i.converged and i.usedIterations == 0 for i in infos) and not x.any()
+    # one opening, where solving the three takes about fifty iterations of 5 us
+    assert sum(t.sampled_ms for t in profiling.read() if t.name == "cg_small") < 0.1
+    b = np.zeros(nrhs * n)
+    b[n:2 * n] = np.random.default_rng(4).standard_normal(n)
+    x = torch.as_tensor(x0.copy(), device=DEV)
+    with resident(finished=1):
+        infos = pa.SolveLinear(A, torch.as_tensor(b, device=DEV), x, maxIterations=4000, tolerance=tol)
+    for k in range(nrhs):
+        xo = x0[k * n:(k + 1) * n].copy()
+        ref = O.cg(row, col, val, b[k * n:(k + 1) * n].copy(), xo, tol, maxit=4000)
+        assert infos[k].converged and abs(infos[k].usedIterations - ref.used_iterations) <= 1 and ref.used_iterations > 10
+        assert np.linalg.norm(x[k * n:(k + 1) * n].cpu().numpy() - xo) <= 2 * np.sqrt(n) * tol / SHIFT
+
+
 @contextmanager
 def no_waiting():
     """Teams of several workgroups give up at the first word that is not there yet."""
