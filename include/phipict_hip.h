@@ -115,6 +115,11 @@ typedef struct pp_csr {
  * remainder on the right-hand side (deferred correction). */
 enum { PP_ADV_CENTRAL = 0, PP_ADV_LINEAR_UPWIND = 1 };
 
+/* pp_domain.corners: MIXED for any domain; DIRECT only if every face is PERIODIC or FIXED and every block has
+ * two or more cells along each axis (no walk is needed); WALKED for any domain, the faster where most
+ * cells lie in a wavefront (64 consecutive cells of a block) with a cell at a connection. */
+enum { PP_CORNERS_MIXED = 0, PP_CORNERS_DIRECT = 1, PP_CORNERS_WALKED = 2 };
+
 typedef struct pp_domain {
     int32_t dims;           /* 2 or 3 */
     int32_t num_blocks;
@@ -142,8 +147,7 @@ typedef struct pp_domain {
     void *scalar_rhs;       /* [batch][C][n] */
     void *scalar_result;    /* [batch][C][n] */
     int32_t advection_scheme; /* PP_ADV_CENTRAL / PP_ADV_LINEAR_UPWIND (Domain::setAdvectionScheme) */
-    int32_t unconnected;    /* 1: every face is PERIODIC or FIXED and every block has two or more cells along
-                             * each axis (lets the corner terms skip the walks); 0: not known */
+    int32_t corners;          /* PP_CORNERS_*: how the corner terms of skewed grids reach the cells around a corner */
 } pp_domain;
 
 /* The reference's LinearSolverResultInfo (csrc/phipict/solvers/linear_solvers.h:180-185). */

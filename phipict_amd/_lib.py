@@ -16,6 +16,7 @@ PP_F32, PP_F64 = 4, 8
 PP_BOUND_CONNECTED, PP_BOUND_PERIODIC, PP_BOUND_FIXED = 20, 21, 30
 PP_BC_DIRICHLET, PP_BC_NEUMANN = 0, 1
 PP_CONV_NORM2, PP_CONV_NORM2_NORMALIZED = 0, 1
+PP_CORNERS_MIXED, PP_CORNERS_DIRECT, PP_CORNERS_WALKED = 0, 1, 2
 
 
 class BoundaryDesc(C.Structure):
@@ -107,7 +108,7 @@ class DomainDesc(C.Structure):
         ("scalar_rhs", C.c_void_p),
         ("scalar_result", C.c_void_p),
         ("advection_scheme", C.c_int32),
-        ("unconnected", C.c_int32),
+        ("corners", C.c_int32),
     ]
 
 

@@ -158,12 +158,23 @@ __device__ __forceinline__ int asm_tile() {
     int p[3];                                                                  \
     unflat(f, b.size, p);
 
-// The template argument NO of the kernels with corner terms: 0 without them, 2 with them for any
-// cell, 1 with them where no cell touches a block connection (the domain says so), without the
-// walks: in one kernel the walks' registers and code burden the cells that never walk. 393 k skewed
-// cells, FP64: advection matrix 109 us with the walks in the kernel, 63 us without (walking 213 us);
-// pressure matrix 80 / 48 (171), momentum right-hand side 74 / 70 (227), divergence 43 / 45 (137).
-static int corner_mode(const pp_domain *dom, int flags) { return flags == 0 ? 0 : (dom->unconnected ? 1 : 2); }
+// The template argument NO of the kernels with corner terms: 0 without them, 1 by direct loads (no cell
+// touches a block connection), 2 by direct loads or walks, wavefront by wavefront, 3 by walks. The domain
+// says which (pp_domain::corners). The walks' registers and code burden the direct loads: 393 k skewed
+// cells of one block, FP64, advection matrix 109 us with the walks in the kernel, 63 us without (walking 213
+// us); pressure matrix 80 / 48 (171), momentum right-hand side 74 / 70 (227), divergence 43 / 45 (137).
+// And the direct loads burden the walks: 131 k cells of three connected blocks 32 and 64 cells wide, where
+// three quarters of the wavefronts walk, FP64, 141 us with both, 127 with the walks alone; a block one cell
+// thick, 90 k cells, 71 and 57 us.
+static int corner_mode(const pp_domain *dom, int flags) {
+    if (flags == 0) return 0;
+    return dom->corners == PP_CORNERS_DIRECT ? 1 : (dom->corners == PP_CORNERS_WALKED ? 3 : 2);
+}
+#define CORNER_KERNEL(K)                                                                                           \
+    (corner_mode(dom, flags) == 0 ? K<T, D, 0>                                                                     \
+                                  : (corner_mode(dom, flags) == 1 ? K<T, D, 1> : (corner_mode(dom, flags) == 2 ? K<T, D, 2> : K<T, D, 3>)))
+template <int NO>
+__device__ __forceinline__ bool take_near(bool ok) { return NO == 1 || (NO == 2 && near_wave(ok)); }
 
 // CSR pattern: row offsets and ascending neighbour columns of every row (shared by the
 // advection, pressure and potential matrices; row layout of topology.cuh:168-233).
@@ -234,9 +245,11 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, i
     for (int k = 0; k < D; ++k) ap[k] = Metric<T, D>::alpha(b, f, k);
     Near<D> nr;
     Cross<T, D> cP;
+    bool near = false;
     if (NO && flags) {
         nr = near_cell<D>(b, p);
-        cP.load(b, f);
+        near = take_near<NO>(nr.ok);
+        if (near) cP.load(b, f);
     }
 #pragma unroll
     for (int bound = 0; bound < 2 * D; ++bound) {
@@ -261,7 +274,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, i
             const T vc = (ap[dim] * vp + an * vn) * T(0.5);
             diag += vc;
             rv[bound + 1] -= vc;
-            if (NO && flags && (NO == 1 || nr.ok)) {
+            if (NO && flags && near) {
                 Cross<T, D> cN;
                 cN.load(b, nf);
                 if (sc < 0) {
@@ -273,7 +286,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_matrix(pp_domain dom, i
                     matrix_corner_near<T, D, NK_SCALAR_TYPES>(cd, bi, nr, p, bound, flags, cP, cN, T(1), T(1), vp, false,
                                                               T(1), diag, rv);
                 }
-            } else if (NO == 2 && flags) {
+            } else if (NO >= 2 && flags) {
                 if (sc < 0) {
                     const CornerData<T, D, NK_VELOCITY_TYPES> cd{dom, blocks, 0, env};
                     matrix_corner_terms<T, D, NK_VELOCITY_TYPES>(cd, bi, p, f, bound, flags, vp, true, nullptr, T(1),
@@ -414,8 +427,8 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_advection_rhs(pp_domain dom, int 
     if (NO && flags) {
         const CornerData<T, D, NK_VELOCITY> cd{dom, blocks, 0, env};
         const Near<D> nr = near_cell<D>(b, p);
-        if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_VELOCITY>(cd, bi, nr, p, f, flags, true, nullptr, Sv);
-        else if constexpr (NO == 2) nonortho_rhs<T, D, NK_VELOCITY>(cd, bi, p, f, flags, true, nullptr, Sv);
+        if (take_near<NO>(nr.ok)) nonortho_rhs_near<T, D, NK_VELOCITY>(cd, bi, nr, p, f, flags, true, nullptr, Sv);
+        else if constexpr (NO >= 2) nonortho_rhs<T, D, NK_VELOCITY>(cd, bi, p, f, flags, true, nullptr, Sv);
     }
 #pragma unroll
     for (int dim = 0; dim < D; ++dim) {
@@ -493,8 +506,8 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_scalar_rhs(pp_domain dom, int fla
             const CornerData<T, D, NK_SCALAR> cd{dom, blocks, ch, env};
             const Near<D> nr = near_cell<D>(b, p);
             T S[1];
-            if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_SCALAR>(cd, bi, nr, p, f, flags, false, nullptr, S);
-            else if constexpr (NO == 2) nonortho_rhs<T, D, NK_SCALAR>(cd, bi, p, f, flags, false, nullptr, S);
+            if (take_near<NO>(nr.ok)) nonortho_rhs_near<T, D, NK_SCALAR>(cd, bi, nr, p, f, flags, false, nullptr, S);
+            else if constexpr (NO >= 2) nonortho_rhs<T, D, NK_SCALAR>(cd, bi, p, f, flags, false, nullptr, S);
             t -= S[0] * scalar_visc<T>(dom, ch);
         }
         rhs[(size_t)ch * dom.num_cells + g] = t / det;
@@ -517,9 +530,11 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_matrix(pp_domain dom, in
     idx[0] = g;
     Near<D> nr;
     Cross<T, D> cP;
+    bool near = false;
     if (NO && flags) {
         nr = near_cell<D>(b, p);
-        cP.load(b, f);
+        near = take_near<NO>(nr.ok);
+        if (near) cP.load(b, f);
     }
 #pragma unroll
     for (int bound = 0; bound < 2 * D; ++bound) {
@@ -538,12 +553,12 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_matrix(pp_domain dom, in
             idx[bound + 1] = ng;
             if (NO && flags) {
                 const CornerData<T, D, NK_FIXED_ONLY> cd{dom, blocks, 0, env};
-                if (NO == 1 || nr.ok) {
+                if (near) {
                     Cross<T, D> cN;
                     cN.load(b, nf);
                     matrix_corner_near<T, D, NK_FIXED_ONLY>(cd, bi, nr, p, bound, flags, cP, cN, raP, raN, T(1), true, T(-1),
                                                             rv[0], rv);
-                } else if constexpr (NO == 2) {
+                } else if constexpr (NO >= 2) {
                     matrix_corner_terms<T, D, NK_FIXED_ONLY>(cd, bi, p, f, bound, flags, raP, false, A, T(1), true, T(-1),
                                                              rv[0], rv);
                 }
@@ -626,8 +641,8 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_pressure_div(pp_domain dom, int t
         const T *A = reinterpret_cast<const T *>(dom.A) + (size_t)env * dom.num_cells;
         const Near<D> nr = near_cell<D>(b, p);
         T S[1];
-        if (NO == 1 || nr.ok) nonortho_rhs_near<T, D, NK_PRESSURE>(cd, bi, nr, p, f, flags, false, A, S);
-        else if constexpr (NO == 2) nonortho_rhs<T, D, NK_PRESSURE>(cd, bi, p, f, flags, false, A, S);
+        if (take_near<NO>(nr.ok)) nonortho_rhs_near<T, D, NK_PRESSURE>(cd, bi, nr, p, f, flags, false, A, S);
+        else if constexpr (NO >= 2) nonortho_rhs<T, D, NK_PRESSURE>(cd, bi, p, f, flags, false, A, S);
         dv += S[0];
     }
     reinterpret_cast<T *>(dom.pressure_rhs_div)[(size_t)env * dom.num_cells + g] = dv;
@@ -1800,7 +1815,7 @@ int pp_setup_advection_matrix(const pp_domain *dom, int32_t non_ortho_flags, voi
     const int flags = matrix_flags(non_ortho_flags);
     PP_CHECK_ARG(dom->C.val && dom->C.row && dom->A && dom->time_step, "C, A and time_step must be set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_ADVECTION_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_matrix<T, D, 1> : k_advection_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, -1, flags))));
+        PP_TIMED(PP_K_ADVECTION_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL(CORNER_KERNEL(k_advection_matrix), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, -1, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1812,7 +1827,7 @@ int pp_setup_advection_matrix_scalar(const pp_domain *dom, int32_t non_ortho_fla
     PP_CHECK_ARG(channel >= 0 && channel < dom->scalar_channels, "passive scalar channel out of range");
     PP_CHECK_ARG(dom->scalar_visc_count == 0 || dom->scalar_viscosity, "scalar viscosity not set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_matrix<T, D, 1> : k_advection_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, (int)channel, flags)));
+        hipLaunchKernelGGL(CORNER_KERNEL(k_advection_matrix), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, (int)channel, flags)));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1824,7 +1839,7 @@ int pp_setup_advection_scalar(const pp_domain *dom, int32_t non_ortho_flags, voi
     PP_CHECK_ARG(!flags || dom->scalar_result, "the non-orthogonal terms read scalar_result");
     PP_CHECK_ARG(dom->scalar_visc_count == 0 || dom->scalar_viscosity, "scalar viscosity not set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_scalar_rhs<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_scalar_rhs<T, D, 1> : k_scalar_rhs<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags)));
+        hipLaunchKernelGGL(CORNER_KERNEL(k_scalar_rhs), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags)));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1835,7 +1850,7 @@ int pp_setup_advection_velocity(const pp_domain *dom, int32_t non_ortho_flags, i
     PP_CHECK_ARG(dom->velocity_rhs && dom->time_step, "velocity_rhs and time_step must be set");
     PP_CHECK_ARG(!flags || dom->velocity_result, "the non-orthogonal terms read velocity_result");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_ADVECTION_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_advection_rhs<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_advection_rhs<T, D, 1> : k_advection_rhs<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_ADVECTION_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL(CORNER_KERNEL(k_advection_rhs), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)apply_pressure_gradient, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
@@ -1846,7 +1861,7 @@ int pp_setup_pressure_matrix(const pp_domain *dom, int32_t non_ortho_flags, void
     const int flags = matrix_flags(non_ortho_flags);
     PP_CHECK_ARG(dom->P.val && dom->P.row && dom->A, "P and A must be set");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_PRESSURE_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_matrix<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_matrix<T, D, 1> : k_pressure_matrix<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags))));
+        PP_TIMED(PP_K_PRESSURE_MATRIX, dom->num_cells, as_stream(stream), hipLaunchKernelGGL(CORNER_KERNEL(k_pressure_matrix), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
 }
@@ -1858,7 +1873,7 @@ int pp_setup_pressure_rhs(const pp_domain *dom, int32_t non_ortho_flags, int32_t
     PP_CHECK_ARG(!flags || (dom->pressure_result && dom->A), "the non-orthogonal terms read pressure_result and A");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
         PP_TIMED(PP_K_PRESSURE_RHS, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((k_pressure_rhs<T, D>), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom));
-        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_div<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_div<T, D, 1> : k_pressure_div<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL(CORNER_KERNEL(k_pressure_div), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)time_step_norm, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;
@@ -1870,7 +1885,7 @@ int pp_setup_pressure_rhs_div(const pp_domain *dom, int32_t non_ortho_flags, int
     PP_CHECK_ARG(dom->pressure_rhs && dom->pressure_rhs_div, "pressure fields must be set");
     PP_CHECK_ARG(!flags || (dom->pressure_result && dom->A), "the non-orthogonal terms read pressure_result and A");
     PP_DISPATCH(dom->dtype, DIMS_DISPATCH(dom->dims,
-        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL((corner_mode(dom, flags) == 0 ? k_pressure_div<T, D, 0> : (corner_mode(dom, flags) == 1 ? k_pressure_div<T, D, 1> : k_pressure_div<T, D, 2>)), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
+        PP_TIMED(PP_K_PRESSURE_DIV, dom->num_cells, as_stream(stream), hipLaunchKernelGGL(CORNER_KERNEL(k_pressure_div), block_grid(dom, dom->batch), dim3(ASM_BLOCK), 0, as_stream(stream), *dom,
                            (int)time_step_norm, flags))));
     PP_LAUNCH_CHECK();
     return PP_OK;

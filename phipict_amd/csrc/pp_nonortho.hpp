@@ -496,6 +496,10 @@ __device__ __forceinline__ Near<D> near_cell(const pp_block_desc &b, const int *
     return n;
 }
 
+// A wavefront takes one way for all its cells: with a cell that needs the walks they all walk, since the
+// wavefront does so in any case.
+__device__ __forceinline__ bool near_wave(bool ok) { return __all(ok) != 0; }
+
 // The cross coefficients alpha_{c1 c2}, c1 < c2, of a cell.
 template <typename T, int D>
 struct Cross {

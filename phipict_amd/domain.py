@@ -1499,9 +1499,28 @@ class Domain:
         d.scalar_rhs = _lib.ptr(self.scalarRHS) if scalar else None
         d.scalar_result = _lib.ptr(self.scalarResult) if scalar else None
         d.advection_scheme = int(self.advectionScheme)
-        d.unconnected = int(all(min(b.getSizesZYX()) > 1 and not any(isinstance(f, ConnectedBoundary) for f in b.boundaries)
-                                for b in self._blocks))
+        d.corners = self._corner_ways()
         self._changed = False
+
+    def _corner_ways(self) -> int:
+        """How the corner terms reach the cells around a corner (``pp_domain.corners``): by direct loads where no
+        cell touches a connection, else by walks where most cells lie in a wavefront (64 consecutive cells) with
+        a cell at a connection. With both ways in a kernel a walk costs ~1.15 times as much as with the
+        walks alone and the direct loads ~0.4 times, so the walks alone are faster above about three quarters."""
+        walked = 0.0
+        for b in self._blocks:
+            sizes = list(reversed(b.getSizesZYX()))
+            if min(sizes) == 1:
+                walked += b.getCells()
+                continue
+            direct = 1.0
+            for a, n in enumerate(sizes):
+                layers = sum(isinstance(f, ConnectedBoundary) for f in b.boundaries[2 * a:2 * a + 2])
+                direct *= 1.0 - min(1.0, layers * (64 if a == 0 else 1) / n)
+            walked += b.getCells() * (1.0 - direct)
+        if walked == 0.0:
+            return _lib.PP_CORNERS_DIRECT
+        return _lib.PP_CORNERS_WALKED if walked > 0.75 * self.totalSize else _lib.PP_CORNERS_MIXED
 
     ATLAS_RING = 16
 
