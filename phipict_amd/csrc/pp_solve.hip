@@ -32,16 +32,16 @@ namespace pp {
 
 // Threads per workgroup of the phase kernels, the level passes and the segmented solves, and of the
 // passes of AMG-PCG over the finest level. Every workgroup folds the partial set that the previous
-// launch left, one value per workgroup: with 512 of them instead of 2048 the three such launches of
-// an iteration over 663 k rows take 32, 23 and 20 us instead of 35, 28 and 22. The CG and BiCGStab
-// kernels share their rows among several right-hand sides and take the registers of one large
-// workgroup per CU: 1.77 M rows of three right-hand sides take 85 us in the small ones, 91 in the
-// large ones.
+// launch left, one value per workgroup: 12 iterations of AMG-PCG on 729 k rows take 3.08 ms with
+// 512 workgroups of 1024 threads, 3.24 with 512 threads, 3.29 with 256 (110 k rows: the same within 5 %).
+// The CG and BiCGStab kernels share their rows among several right-hand sides and take the registers of
+// one large workgroup per CU: 1.77 M rows of three right-hand sides take 85 us in the small ones, 91
+// in the large ones.
 constexpr int WG = 256;
 constexpr int PCG_WG = 1024;
-// Threads per CU of the phase kernels and of the level passes (a half, three eighths and a quarter
-// measured the same or slower: 663 k rows of AMG-PCG 7.39, 7.30 and 7.53 ms for 7.23, BiCGStab on
-// 1.77 M rows 1.34, 1.42 and 2.09 ms for 0.96).
+// Threads per CU of the phase kernels and of the level passes. With a half, 12 iterations of BiCGStab on
+// 1.77 M rows of three right-hand sides take 5.5 ms instead of 3.9, of AMG-PCG on 729 k rows 2.98 instead
+// of 3.08, on 110 k rows 1.62 instead of 1.54.
 constexpr int PHASE_THREADS = 2048;
 
 // ======================================================================================
@@ -109,8 +109,8 @@ __device__ __forceinline__ void fold(const Parts &P, int q0, int first, int coun
 }
 
 // What a phase kernel's first wavefront decided, for the others: one wavefront folds and applies the
-// rules, several hundred straight instructions that all of them executed before (BiCGStab on 1.77 M
-// rows of three right-hand sides: 958 us with it, 984 without).
+// rules, several hundred straight instructions, instead of all of them (BiCGStab on 1.77 M rows of
+// three right-hand sides, records then still copied as blocks: 958 us with it, 984 without).
 template <int NB, typename T>
 struct Head {
     double tot[NB * 3], tot2[NB * 3]; // folded sums
@@ -1720,13 +1720,16 @@ private:
 // How a resident solve of `teams` systems of n rows runs: one workgroup each, or teams of G
 // workgroups with R rows per thread, `perLaunch` teams at a time. ew 0: not on this engine.
 //
-// Measured, us per CG iteration in FP64 (the multi-launch engine: 42 at 160 k rows, 36 at 105 k; the
-// one-workgroup engine: 24 at 4 k rows and growing with the rows):
-//   one workgroup:     1 k rows 1.7, 3 k 2.1, 4 k (five entries) 2.9, 3 k (seven) 2.5
-//   teams, R = 1:      4 k 3.9, 8 k 4.2, 31 k 4.8 (five); 31 k 5.0, 105 k 7.1 (seven)
-//   teams, R = 2:      8 k 4.6, 31 k 4.9; 31 k 5.8, 105 k 7.4, 160 k 8.7, 246 k 9.3
-//   teams, R = 4:      8 k 5.5, 31 k 6.8; 31 k 9.8, 105 k 11.9, 246 k 15
-// so one workgroup as long as its registers hold the rows, then the fewest rows per thread
+// Measured, us per CG iteration in FP64, five / seven entries per row:
+//   one workgroup:     1 k rows 1.8, 3 k 2.2 / 2.5, 4 k 3.0 (five; the one-workgroup engine 24)
+//   teams, R = 1:      4 k 4.1, 8 k 4.4, 31 k 4.9 / 5.4, 66 k 5.2, 108 k - / 7.2, 131 k 7.0
+//   teams, R = 2:      160 k - / 9.1, 262 k 8.4 / 9.1
+//   teams, R = 4:      360 k 12.1, 343 k - / 17.3, 524 k 14.0 / 21.5
+// with R larger than the rows need: 31 k 4.9 / 5.8 (R = 2), 6.8 / 9.8 (R = 4); 105 k - / 7.4, - / 11.9.
+// The multi-launch engine: 34 k 10.9 / 11.5, 108 k - / 13.1, 131 k 13.2, 262 k 17.8 / 16.0, 343 k - / 22.9,
+// 524 k 28.6 / 29.6; several right-hand sides of one matrix, which share its rows there: 262 k of
+// seven entries x 2 25.4 (teams 20.4), 108 k x 4 29.0 (16.3), 131 k of five x 4 27.8 (10.5).
+// So one workgroup as long as its registers hold the rows, then the fewest rows per thread
 // that let all teams run at once; if none does, as many teams at a time as fit with R = 4.
 struct ResPlan {
     int ew = 0, R = 0, threads = 0, G = 1, perLaunch = 0;
@@ -2652,6 +2655,10 @@ static int upload_layout(SegSpace &sg, const std::vector<int32_t> &host, hipStre
 // one-workgroup teams (`local` of them). Chosen among R = 1, 2, 4 by the time of the launches, each its
 // longest piece's iterations (about the root of its rows) times the time of one (measured at
 // 8 k - 31 k rows, us): fewer rows per thread iterate faster and need more launches.
+// Beside the engine of tiles, us per iteration in FP64: 12 pieces of 5 k rows x 2 4.5 (tiles 17), 64 of 8 k of
+// seven entries 17 (33), 200 of 10 k 33 (69), 400 of 4 k of seven entries 43 (58), 6 of 250 k 36 (47). Where large
+// pieces of seven entries need many launches the two meet: 24 of 64 k 55 (53), 2 of 512 k 42 (42), 6 of 216 k
+// 59 (47). All go to the teams, whose time is that of the longest piece of each launch alone.
 struct SegPack {
     int R = 0, localR = 0, launches = 0;          // launches of teams
     double cost = 0.0;
