@@ -268,9 +268,10 @@ struct Rows {
     }
 };
 
+// Past the L2 cache of the workgroup's XCD, like the exchanged words: workgroups on other XCDs look at it.
 template <typename T>
 __device__ __forceinline__ void give_up(const ResArgs<T> &a) {
-    if (threadIdx.x == 0) *a.failed = a.done;
+    if (threadIdx.x == 0) __hip_atomic_store(a.failed, a.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Rows longer than the resident kernels take. They are looked for before anything is solved: pieces that
